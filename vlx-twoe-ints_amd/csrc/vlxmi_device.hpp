@@ -199,4 +199,39 @@ __device__ __forceinline__ void boys_lds(double T, const double* lt, double* F)
     }
 }
 
+// The N-point Rys rule of argument T (tables and their accuracy:
+// vlxmi/gen/rys.py): roots times ``su`` to slot[i * 64], weights times ``sw``
+// to slot[(N + i) * 64], i < N -- lane-private LDS slots, so that the kernels'
+// point loops index them at run time.  T < 64: one degree-7 polynomial per
+// value on intervals of width 1/4 (64 contiguous bytes per lane and value);
+// above, the half-range Gauss-Hermite rule scaled by T.
+#define VLX_RYS_TMAX 64.0
+#define VLX_RYS_INV_WIDTH 4.0
+#define VLX_RYS_NCOEF 8
+
+template <int N>
+__device__ __forceinline__ void rys_points(double T, const double* __restrict__ table, const double* large, double su,
+                                           double sw, double* slot)
+{
+    if (T < VLX_RYS_TMAX) {
+        const int k = (int)(T * VLX_RYS_INV_WIDTH);
+        const double x = T * (2.0 * VLX_RYS_INV_WIDTH) - (double)(2 * k + 1);
+        const double* c = table + k * (2 * N * VLX_RYS_NCOEF);
+#pragma unroll
+        for (int f = 0; f < 2 * N; ++f) {
+            double s = c[f * VLX_RYS_NCOEF + VLX_RYS_NCOEF - 1];
+#pragma unroll
+            for (int j = VLX_RYS_NCOEF - 2; j >= 0; --j) s = fma(s, x, c[f * VLX_RYS_NCOEF + j]);
+            slot[f * 64] = s * (f < N ? su : sw);
+        }
+    } else {
+        const double y = rsq_nr(T), ty = su * (y * y), wy = sw * y;
+#pragma unroll
+        for (int f = 0; f < N; ++f) {
+            slot[f * 64] = large[f] * ty;
+            slot[(N + f) * 64] = large[N + f] * wy;
+        }
+    }
+}
+
 }  // namespace vlxmi

@@ -35,6 +35,7 @@ import time
 
 from . import emit
 from . import emit_grad
+from . import rys as ryspts
 from ..pairs import PAIR_CLASSES, j_classes, k_classes
 
 PKG = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))   # vlx-twoe-ints_amd
@@ -66,29 +67,30 @@ BOYS_LDS_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "boys_
 # LDS Boys rows), chosen from per-class timings
 WPG_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "wpg.json")
 
-# heavy exchange classes whose plain FP64 kernel runs one pass per ket
-# component pair (emit.emit_k kpairs), chosen from lattice64 per-class timings
-K_PASSES_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "k_passes.json")
+# classes whose FP64 kernels evaluate the quartets by Rys quadrature instead of
+# the Head-Gordon-Pople recursion, per kernel kind (J, K: class launchers and
+# their batched variants; JG, KG: gradients), with the component sums per pass
+# and the place of the thresholds; chosen from per-class timings (the file's
+# _doc)
+RYS_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "rys.json")
+RYS_KINDS = ("J", "K", "JG", "KG")
 
 
-J_PASSES_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "j_passes.json")
+def load_rys():
+    """{kind: {class: {"maxx", "tau", "waves"}}}."""
+    tab = {}
+    if os.path.exists(RYS_TABLE):
+        with open(RYS_TABLE) as f:
+            tab = json.load(f)
+    return {kind: {cls: dict(zip(("maxx", "tau", "waves"), v)) for cls, v in tab.get(kind, {}).items()}
+            for kind in RYS_KINDS}
 
 
-def _pair_classes(path):
-    if not os.path.exists(path):
-        return set()
-    with open(path) as f:
-        return {k for k, v in json.load(f).items() if not k.startswith("_") and v == "pair"}
-
-
-def load_k_passes():
-    """Classes whose plain FP64 exchange kernel runs pair passes."""
-    return _pair_classes(K_PASSES_TABLE)
-
-
-def load_j_passes():
-    """Split Coulomb classes whose plain FP64 kernel runs pair passes."""
-    return _pair_classes(J_PASSES_TABLE)
+# Coulomb bra classes with many blocks: a tile is full but for the list's last
+# one, so sharing the lanes of short tiles out among ket records gains nothing
+# there and its two instructions a record cost the light classes 2-5 %
+# (lattice of 48 atoms: (ss|sp) 12.3 -> 12.9 ms)
+J_UNPACKED = ("ss", "sp")
 
 
 # gradient classes whose kernels run one pass per ket-first-index component
@@ -98,18 +100,19 @@ GRAD_PASSES_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gr
 
 
 def grad_k_layout(gp, cls):
-    """(passes, split) of the exchange-gradient kernel of ``cls``."""
-    v = gp["K"].get(cls, "one")
-    return (v[len("split_"):], True) if v.startswith("split_") else (v, False)
+    """(passes, split) of the exchange-gradient recursion of ``cls``; no class
+    is split by centre any more (the second value is always False)."""
+    return gp["K"].get(cls, "one"), False
 
 
 def load_grad_passes():
-    """{"J": {class: passes}, "K": {class: passes}}; absent classes run one pass."""
+    """{"J": {class: passes}, "K": {class: passes}, "centres": classes with
+    one-centre kernels beside the class's own}; absent classes run one pass."""
     tab = {}
     if os.path.exists(GRAD_PASSES_TABLE):
         with open(GRAD_PASSES_TABLE) as f:
             tab = json.load(f)
-    return {k: dict(tab.get(k, {})) for k in ("J", "K")}
+    return dict({k: dict(tab.get(k, {})) for k in ("J", "K")}, centres=set(tab.get("centres", [])))
 
 
 FAMILIES = ("J", "K", "Jb", "Kb")     # class launchers (+ _mixed), batched (+ _mixed)
@@ -159,6 +162,11 @@ def load_layouts(path=None):
     return {}
 
 
+def rys_inc(cls, extra, r):
+    """Table include of a Rys kernel (``extra`` orders above the class's own)."""
+    return emit.rys_include(sum(emit.LV[x] for x in cls) + extra) if r else ""
+
+
 def sources(tiles=None, layouts=None):
     """Map file name -> source text of every generated translation unit."""
     tiles = load_tiles() if tiles is None else tiles
@@ -169,31 +177,37 @@ def sources(tiles=None, layouts=None):
     wpg = load_wpg()
     out = {}
     inc = '#include "vlxmi_device.hpp"\n\n'
-    jpairs = load_j_passes()
+    rys = load_rys()
     for ab, cd in j_classes():
         cls = j_name(ab, cd)
-        for pre, kw in (("j", dict(jpairs=cls in jpairs)), ("jm", dict(mixed=True)), ("jb", dict(batched=True)),
+        for pre, kw in (("j", {}), ("jm", dict(mixed=True)), ("jb", dict(batched=True)),
                         ("jbm", dict(batched=True, mixed=True))):
             fn = "%s_%s.hip" % (pre, cls)
             fam = "Jb" if kw.get("batched") else "J"
-            out[fn] = inc + emit.emit_j(cls, kt=tiles.get(fn), layout=jlayouts.get(cls, "reg"),
-                                        lds_boys=cls in blds[fam], wpg=int(wpg[fam].get(cls, 1)), **kw)
-    kpairs = load_k_passes()
+            r = None if kw.get("mixed") else rys["J"].get(cls)
+            out[fn] = rys_inc(cls, 0, r) + inc + emit.emit_j(
+                cls, kt=tiles.get(fn), layout=jlayouts.get(cls, "reg"), lds_boys=cls in blds[fam],
+                wpg=int(wpg[fam].get(cls, 1)), rys=r, pack=ab not in J_UNPACKED, **kw)
     for cls in k_classes():
-        for pre, kw in (("k", dict(kpairs=cls in kpairs)), ("km", dict(mixed=True)), ("kb", dict(batched=True)),
+        for pre, kw in (("k", {}), ("km", dict(mixed=True)), ("kb", dict(batched=True)),
                         ("kbm", dict(batched=True, mixed=True))):
             fn = "%s_%s.hip" % (pre, cls)
             fam = "Kb" if kw.get("batched") else "K"
-            out[fn] = inc + emit.emit_k(cls, kt=tiles.get(fn), layout=layouts.get(cls, "reg"),
-                                        dorder=dorders.get(cls, "jl"), lds_boys=cls in blds[fam],
-                                        wpg=int(wpg[fam].get(cls, 1)), **kw)
+            r = None if kw.get("mixed") else rys["K"].get(cls)
+            out[fn] = rys_inc(cls, 0, r) + inc + emit.emit_k(
+                cls, kt=tiles.get(fn), layout=layouts.get(cls, "reg"), dorder=dorders.get(cls, "jl"),
+                lds_boys=cls in blds[fam], wpg=int(wpg[fam].get(cls, 1)), rys=r, pack=True, **kw)
     gp = load_grad_passes()
     for ab, cd in j_classes():
         cls = j_name(ab, cd)
-        out["jg_%s.hip" % cls] = inc + emit_grad.emit_jgrad(cls, passes=gp["J"].get(cls, "one"))
+        r = rys["JG"].get(cls)
+        out["jg_%s.hip" % cls] = rys_inc(cls, 1, r) + inc + emit_grad.emit_jgrad(cls, passes=gp["J"].get(cls, "one"), rys=r)
     for cls in k_classes():
-        passes, split = grad_k_layout(gp, cls)
-        out["kg_%s.hip" % cls] = inc + emit_grad.emit_kgrad(cls, passes=passes, split=split)
+        r = rys["KG"].get(cls)
+        out["kg_%s.hip" % cls] = rys_inc(cls, 1, r) + inc + emit_grad.emit_kgrad(
+            cls, passes=grad_k_layout(gp, cls)[0], rys=r, centres=cls in gp["centres"])
+    for n in range(1, ryspts.NMAX + 1):
+        out["rys_table_%d.h" % n] = ryspts.header_text(n)
     for pc in PAIR_CLASSES:
         out["schwarz_%s.hip" % pc] = inc + emit.emit_schwarz(pc)
     out["jdispatch.hip"] = inc + jdispatch_text()
@@ -279,19 +293,18 @@ def device_header_text():
           " *   computeCoulombGradient{AB}{CD}: blockDim 64, gridDim (ceil(bra blocks / 64), ket chunks);",
           " *     chunk y stores the six sums of bra block bb at grad[(y * nbra + bb) * 6 + 0..5];",
           " *   computeExchangeGradient{A}{B}{C}{D}: blockDim 64, gridDim = (i,k) blocks; adds six sums",
-          " *     per block to grad[blk * 6 + 0..5]; for the classes split by centre, the _A kernel adds",
-          " *     columns 0..2 and the _C kernel columns 3..5 (the launcher runs both). */"]
+          " *     per block to grad[blk * 6 + 0..5]; where declared, the _A kernel adds only columns 0..2",
+          " *     and the _C kernel only columns 3..5. */"]
     for ab, cd in j_classes():
         cls = j_name(ab, cd)
         o.append("__global__ void computeCoulombGradient%s(%s);" % (cls.upper(), ", ".join(emit._strip_restrict(emit_grad.jg_signature(cls)))))
     gp = load_grad_passes()
     for cls in k_classes():
         sig = ", ".join(emit._strip_restrict(emit_grad.kg_signature(cls)))
-        if grad_k_layout(gp, cls)[1]:
+        o.append("__global__ void computeExchangeGradient%s(%s);" % (cls.upper(), sig))
+        if cls in gp["centres"]:
             o.append("__global__ void computeExchangeGradient%s_A(%s);" % (cls.upper(), sig))
             o.append("__global__ void computeExchangeGradient%s_C(%s);" % (cls.upper(), sig))
-        else:
-            o.append("__global__ void computeExchangeGradient%s(%s);" % (cls.upper(), sig))
     o += ["", "#endif", ""]
     return "\n".join(o)
 
@@ -570,12 +583,15 @@ def _build(jobs=None, force=False, only=None, verbose=True):
         objs.append(o)
         if force or not os.path.exists(o):
             todo.append((p, o, ("-x", "hip")))
+    dev_hdr += "".join(text for fn, text in sorted(srcs.items()) if fn.endswith(".h"))
     for fn, text in srcs.items():
         p = os.path.join(GEN, fn)
         old = open(p).read() if os.path.exists(p) else None
         if old != text:
             with open(p, "w") as f:
                 f.write(text)
+        if fn.endswith(".h"):
+            continue
         h = hashlib.sha1((text + dev_hdr + flag_key).encode()).hexdigest()[:16]
         o = os.path.join(OBJ, "%s.%s.o" % (fn, h))
         objs.append(o)

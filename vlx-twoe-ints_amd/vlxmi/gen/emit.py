@@ -28,7 +28,9 @@ Schwarz: one lane per primitive-pair block computes the (ab|ab) diagonal.
 
 from __future__ import annotations
 
+from . import rys as ryspts
 from .osdag import QuartetDAG, tri
+from .rysdag import RysPoint
 
 LV = {"s": 0, "p": 1, "d": 2}
 NC = {"s": 1, "p": 3, "d": 6}
@@ -117,6 +119,88 @@ def launder(L):
         grp = names[i:i + 10]
         out.append('asm volatile("" : %s);' % ", ".join('"+v"(%s)' % n for n in grp))
     return out
+
+
+# --------------------------------------------------------------------------
+# Rys quadrature bodies
+# --------------------------------------------------------------------------
+
+def rys_groups(nab, nc, nd, maxx):
+    """Passes over the ket component pairs (ic, id) of at most ``maxx``
+    component sums (nab per pair, a register pair each; at least one pair):
+    whole second-index components id where they fit, else equal shares of the
+    first-index components of one id -- an exchange pass then gathers only the
+    density elements of its own id."""
+    per = max(1, maxx // nab)
+    if per >= nc:
+        k = max(x for x in range(1, nd + 1) if nd % x == 0 and x * nc <= per)
+        return [[(ic, idd) for idd in range(g * k, (g + 1) * k) for ic in range(nc)] for g in range(nd // k)]
+    k = max(x for x in range(1, nc + 1) if nc % x == 0 and x <= per)
+    return [[(ic, idd) for ic in range(g * k, (g + 1) * k)] for idd in range(nd) for g in range(nc // k)]
+
+
+def rys_include(L):
+    """Include of the table the points of total order L are read from."""
+    return '#include "rys_table_%d.h"\n\n' % ryspts.nroots(L)
+
+
+def rys_decl(L, wpg=1):
+    """LDS slots of one wavefront's quadrature points ([u_0.., w_0..][lane])."""
+    n = ryspts.nroots(L)
+    return ["    __shared__ double lrys_all[%d * %d];" % (wpg, 2 * n * 64),
+            "    double* lrys = lrys_all + %slane;" % ("" if wpg == 1 else "wave * %d + " % (2 * n * 64))]
+
+
+def rys_prologue(L, omega=False, ind="    "):
+    """As quartet_prologue, with the roots u_i (times the attenuation) and the
+    weights w_i Lambda of the quartet in the lane's LDS slots instead of
+    Lambda-scaled Boys values in registers."""
+    n = ryspts.nroots(L)
+    o = quartet_prologue(0, omega=omega, ind="")
+    k = [i for i, x in enumerate(o) if x.startswith("double Fb[")][0]
+    del o[k:k + 3]                       # Fb, its evaluation, F0
+    o.insert(k, "vlxmi::rys_points<%d>(Tb, vlxmi::rys_table_%d, vlxmi::rys_large_%d, %s, Lambda, lrys);"
+             % (n, n, n, "d2" if omega else "1.0"))
+    return [ind + x for x in o]
+
+
+def rys_pass(la, lb, lc, ld, group, prefix, ind):
+    """One pass: X{tab}_{tcd} = sum over the points of Ix Iy Iz for every bra
+    component pair tab and the ket pairs of ``group``.  The points run in a
+    loop that is not unrolled: one point's one-dimensional integrals are live
+    at a time and the kernel's code stays within the instruction cache."""
+    nb, nd = NC["spd"[lb]], NC["spd"[ld]]
+    n = ryspts.nroots(la + lb + lc + ld)
+    pt = RysPoint(prefix=prefix)
+    names, sums = [], []
+    for ic, idd in group:
+        for ia, aa in enumerate(tri(la)):
+            for ib, bb in enumerate(tri(lb)):
+                x = "X%d_%d" % (ia * nb + ib, ic * nd + idd)
+                names.append(x)
+                pt.lines.append("%s += %s;" % (x, pt.component(aa, bb, tri(lc)[ic], tri(ld)[idd])))
+    o = [ind + "double %s;" % ", ".join(x + " = 0.0" for x in names)]
+    loop = [ind + "    const double ru = lrys[ir * 64], rw = lrys[(%d + ir) * 64];" % n]
+    loop += [ind + "    " + x for x in pt.lines]
+    if n == 1:
+        return o + [ind + "{", ind + "    constexpr int ir = 0;"] + loop + [ind + "}"]
+    return o + [ind + "#pragma unroll 1", ind + "for (int ir = 0; ir < %d; ++ir) {" % n] + loop + [ind + "}"]
+
+
+def rys_grad_pass(la, lb, lc, ld, group, cents, prefix, ind):
+    """One gradient pass: the point loop over the component weights
+    W{tab}_{tcd} (declared by the caller) of the ket pairs of ``group``."""
+    nb, nd = NC["spd"[lb]], NC["spd"[ld]]
+    n = ryspts.nroots(la + lb + lc + ld + 1)
+    pt = RysPoint(prefix=prefix)
+    pt.gradient_terms([("W%d_%d" % (ia * nb + ib, ic * nd + idd), aa, bb, tri(lc)[ic], tri(ld)[idd])
+                       for ic, idd in group for ia, aa in enumerate(tri(la)) for ib, bb in enumerate(tri(lb))],
+                      cents, "gacc")
+    loop = [ind + "    const double ru = lrys[ir * 64], rw = lrys[(%d + ir) * 64];" % n]
+    loop += [ind + "    " + x for x in pt.lines]
+    if n == 1:
+        return [ind + "{", ind + "    constexpr int ir = 0;"] + loop + [ind + "}"]
+    return [ind + "#pragma unroll 1", ind + "for (int ir = 0; ir < %d; ++ir) {" % n] + loop + [ind + "}"]
 
 
 def _live_estimate(la, lb, lc, ld, cgroup):
@@ -227,19 +311,50 @@ def _dag_lines(dag):
     return out
 
 
-def ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=False):
+def pack_decls(ind, rem, lane="lane"):
+    """How a tile's lanes are shared out in a packed kernel: the largest power
+    of two W of bra blocks that is not mostly empty takes the wavefront's
+    lanes, which form G = 64 / W groups; group ``slot`` of lanes evaluates
+    every G-th ket record.  ``rem`` is the (uniform) number of blocks left.
+    W is the power of two that holds ``rem`` (at most 64), halved when the
+    blocks would fill at most three quarters of it: the rest then follow in a
+    narrower tile."""
+    return [ind + "uint32_t wsh = %s > 32 ? 6 : (%s > 1 ? 32 - __clz(%s - 1) : 0);" % (rem, rem, rem),
+            ind + "if (wsh > 3 && %s * 4 <= (3u << wsh)) --wsh;" % rem,
+            ind + "const uint32_t slot = %s >> wsh, G = 64u >> wsh, jl = %s & ((1u << wsh) - 1);" % (lane, lane)]
+
+
+def pack_decls1(ind, rem):
+    """As pack_decls for a kernel whose tile is fixed (a Coulomb bra tile of at
+    most 64 blocks): W is the power of two that holds ``rem`` blocks."""
+    return [x for x in pack_decls(ind, rem) if "--wsh" not in x]
+
+
+def ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=False, pack=False):
     """One loop over the staged records from the current ``s`` to nt-1, the
     recursion in type ``ty``; with ``check_lo`` it stops (setting ``lo``) at
     the first record where every live lane's bound is below fp32_threshold.
     With ``count`` every evaluated quartet adds one to the lane's counter of
-    its precision (nq64 / nq32)."""
-    q = [ind + "for (; s < nt; ++s) {",
-         ind + "    const double* R = ket + s * REC;",
-         ind + "    if (%s && %s) %s = false;" % (act, screen, act),
-         ind + "    if (!__any(%s)) break;" % act]
+    its precision (nq64 / nq32).  Packed: the lane groups take records sb,
+    sb + 1, .. sb + G - 1 (the lanes of a group beyond the tile's end wait)."""
+    if pack:
+        q = [ind + "for (; sb < nt; sb += G) {",
+             ind + "    const uint32_t s = sb + slot < nt ? sb + slot : sb;",
+             ind + "    const double* R = ket + s * REC;",
+             ind + "    bool live = %s && sb + slot < nt;" % act,
+             ind + "    if (live && %s) live = %s = false;" % (screen, act)]
+    else:
+        q = [ind + "for (; s < nt; ++s) {",
+             ind + "    const double* R = ket + s * REC;",
+             ind + "    if (%s && %s) %s = false;" % (act, screen, act)]
+    live = "live" if pack else act
+    q.append(ind + "    if (!__any(%s)) break;" % act)
     if check_lo:
-        q.append(ind + "    if (__all(!%s || %s < fp32_threshold)) { %s = true; break; }" % (act, bound, lo))
-    q.append(ind + "    if (%s) {" % act)
+        # packed: a group past the tile's end says nothing about its next record,
+        # but the lanes of group 0 hold the same bra blocks and larger bounds
+        q.append(ind + "    if (%s__all(!%s || %s < fp32_threshold)) { %s = true; break; }"
+                 % ("__any(live) && " if pack else "", live, bound, lo))
+    q.append(ind + "    if (%s) {" % live)
     if count:
         q.append(ind + "        %s += 1u;" % ("nq32" if ty == "float" else "nq64"))
     q += [ind + "        " + x for x in header]
@@ -248,7 +363,22 @@ def ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=Fals
     return q
 
 
-def ket_loops(ind, act, screen, bound, header, body, mixed, lo, count=None):
+def rys_ket_loop(ind, screen, header, body, count=False):
+    """The (packed) ket loop of a Rys kernel: the whole wavefront runs the
+    quartets; the body masks what it adds by the lane's flag ``live``."""
+    q = [ind + "for (uint32_t sb = 0; sb < nt; sb += G) {",
+         ind + "    const uint32_t s = sb + slot < nt ? sb + slot : sb;",
+         ind + "    const double* R = ket + s * REC;",
+         ind + "    bool live = active && sb + slot < nt;",
+         ind + "    if (live && %s) live = active = false;" % screen,
+         ind + "    if (!__any(active)) break;"]
+    if count:
+        q.append(ind + "    nq64 += live ? 1u : 0u;")
+    q += [ind + "    " + x for x in header]
+    return q + body("double", ind + "    ") + [ind + "}"]
+
+
+def ket_loops(ind, act, screen, bound, header, body, mixed, lo, count=None, pack=False):
     """Loop(s) over the staged ket records s = 0..nt-1 of one tile.
 
     ``act`` is the lane's live flag, cleared by the screening test ``screen``
@@ -263,9 +393,9 @@ def ket_loops(ind, act, screen, bound, header, body, mixed, lo, count=None):
     count = mixed if count is None else count
 
     def loop(ty, check_lo):
-        return ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=count)
+        return ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=count, pack=pack)
 
-    o = [ind + "{", ind + "uint32_t s = 0;"]
+    o = [ind + "{", ind + "uint32_t %s = 0;" % ("sb" if pack else "s")]
     if mixed:
         o.append(ind + "if (!%s) {" % lo)
         o += ["    " + x for x in loop("double", True)]
@@ -403,15 +533,23 @@ def ket_record_bytes(kind, cls):
     return rec * 8 + (NC[d] * 4 if kind == "K" else 0)
 
 
-def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=False, wpg=1, jpairs=False):
+def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=False, wpg=1, jpairs=False, rys=None,
+           pack=False):
     """Source of computeCoulombFock{CLS} (or its _mixed / _batched variants) and its
     C-ABI launcher.  The batched variant is persistent: workgroup w processes
     work items w, w + gridDim.x, ...; item t = (bra block begin, bra block end
     (<= begin + 64), ket block begin, ket block end) over lists that concatenate
-    many molecules; each bra tile must appear in at most one item (plain +=)."""
+    many molecules; each bra tile must appear in at most one item (plain +=).
+    ``rys`` ({"maxx", "tau", "waves"}, FP64 only): evaluate the quartet by Rys
+    quadrature in passes of at most ``maxx`` component sums; "tau" says where
+    the accumulators and thresholds are kept ("reg" or "lds"), "waves" the
+    wavefronts per SIMD the registers are allotted for.  ``pack``: a tile of
+    few bra blocks shares its lanes out among several ket records (pack_decls;
+    Rys kernels always do)."""
     a, b, c, d = cls
     la, lb, lc, ld = LV[a], LV[b], LV[c], LV[d]
     na, nb, nc, nd = NC[a], NC[b], NC[c], NC[d]
+    pack = pack or rys is not None
     ab, cd = a + b, c + d
     nab, ncd = na * nb, nc * nd
     L = la + lb + lc + ld
@@ -428,7 +566,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     # partial sums at ket_partial[y * count_local + e] for the launcher's
     # deterministic reduction.
     KP = ["double* __restrict__ ket_partial"]
-    LB = "TILE_SIZE_J" if wpg == 1 else str(64 * wpg)
+    LB = ("TILE_SIZE_J" if wpg == 1 else str(64 * wpg)) + (", %d" % rys["waves"] if rys and rys.get("waves") else "")
     if batched:
         o.append("__global__ void __launch_bounds__(%s)" % LB)
         o.append("%s(%s)" % (name, ",\n    ".join(sig)))
@@ -448,6 +586,8 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         o.append("    double* ket = ket_all + wave * (KT * REC);")
     if lds_boys:
         o += lds_boys_setup(L)
+    if rys:
+        o += rys_decl(L, wpg)
     o.append("    const uint32_t nbra = %s_prim_pair_count_local / NAB;" % ab)
     o.append("    const uint32_t nket = %s_prim_pair_count / NCD;" % cd)
     if batched:
@@ -457,12 +597,18 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         else:
             o.append("    for (uint32_t w = blockIdx.x * WPG + wave; w < nwork; w += gridDim.x * WPG) {")
         o.append("    const uint32_t bra_end = work[4 * w + 1] < nbra ? work[4 * w + 1] : nbra;")
-        o.append("    const uint32_t bb = work[4 * w] + lane;")
+        if pack:
+            o += pack_decls1("    ", "(bra_end - work[4 * w])")
+        o.append("    const uint32_t bb = work[4 * w] + %s;" % ("jl" if pack else "lane"))
         o.append("    const uint32_t k_begin = work[4 * w + 2];")
         o.append("    const uint32_t k_end = work[4 * w + 3] < nket ? work[4 * w + 3] : nket;")
         o.append("    const bool own = bb < bra_end;")
     else:
-        o.append("    const uint32_t bb = %s * TILE_SIZE_J + lane;" % ("blockIdx.x" if wpg == 1 else "(blockIdx.x * WPG + wave)"))
+        tile = "blockIdx.x" if wpg == 1 else "(blockIdx.x * WPG + wave)"
+        if pack:
+            o.append("    const uint32_t left = nbra > %s * TILE_SIZE_J ? nbra - %s * TILE_SIZE_J : 0;" % (tile, tile))
+            o += pack_decls1("    ", "left")
+        o.append("    const uint32_t bb = %s * TILE_SIZE_J + %s;" % (tile, "jl" if pack else "lane"))
         o.append("    const uint32_t chunk = (nket + gridDim.y - 1) / gridDim.y;")
         o.append("    const uint32_t k_begin = blockIdx.y * chunk;")
         o.append("    const uint32_t k_end = (k_begin + chunk < nket) ? (k_begin + chunk) : nket;")
@@ -471,8 +617,12 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("    bool active = own;")
     o.append("    double zeta = 1.0, sq_zeta = 1.0, inv_S1 = 1.0, P_x = 0.0, P_y = 0.0, P_z = 0.0;")
     o.append("    double PA_x = 0.0, PA_y = 0.0, PA_z = 0.0, AB_x = 0.0, AB_y = 0.0, AB_z = 0.0;")
-    o.append("    double qmax = 0.0;")
+    o.append("    double qmax = 0.0%s;" % (", taumax = 0.0" if rys else ""))
     jsl = plan_slices(la, lb, lc, ld, "J")
+    if rys:
+        assert not mixed, "Rys bodies are for the FP64 kernels"
+        layout, lds_boys, jpairs = rys["tau"], False, False
+        jsl = rys_groups(nab, nc, nd, rys["maxx"])
     if len(jsl) > 1 and jpairs:
         # one pass per ket component pair (ic, id), recursion recomputed per pair
         assert not mixed, "pair passes are for the FP64 kernels"
@@ -482,7 +632,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     # "lds" keeps them in LDS ([component][lane], lane-private slots), the
     # digestion adding each term with one LDS f64 add and reading the
     # threshold per use, which frees 4*NAB registers for the recursion.
-    jlds = len(jsl) > 1 and layout == "lds"
+    jlds = (len(jsl) > 1 or rys is not None) and layout == "lds"
     assert not (jlds and wpg > 1), "the LDS accumulator layout keeps one wavefront per workgroup"
     if jlds:
         o.append("    __shared__ double ltau[NAB * TILE_SIZE_J], lacc[NAB * TILE_SIZE_J];")
@@ -511,6 +661,9 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("            const double q = fabs(%s_mat_Q_local[e0 + t]);" % ab)
     o.append("            qmax = fmax(qmax, q);")
     o.append("            tau[%s] = thr / q;" % ("t * TILE_SIZE_J + lane" if jlds else "t"))
+    if rys:
+        # 0/0 (a zero bound at a zero threshold) passes nothing, like infinity
+        o.append("            if (%s_pair_data_local[e0 + t] != 0.0) taumax = fmax(taumax, thr / q >= 0.0 ? thr / q : __builtin_inf());" % ab)
     o.append("        }")
     o.append("    }")
     if mixed:
@@ -536,7 +689,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("                R[3] = (ak * C_x + al * D_x) * iet; R[4] = (ak * C_y + al * D_y) * iet; R[5] = (ak * C_z + al * D_z) * iet;")
     o.append("                R[6] = (al * iet) * (D_x - C_x); R[7] = (al * iet) * (D_y - C_y); R[8] = (al * iet) * (D_z - C_z);")
     o.append("                R[9] = C_x - D_x; R[10] = C_y - D_y; R[11] = C_z - D_z;")
-    o.append("                double beta = 0.0;")
+    o.append("                double beta = 0.0%s;" % (", qmin = __builtin_inf()" if rys else ""))
     o.append("                #pragma unroll")
     o.append("                for (int t = 0; t < NCD; ++t) {")
     o.append("                    const double Dkl = %s_mat_D[f0 + t];" % cd)
@@ -548,7 +701,12 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("                    const double qd = fabs(%s_mat_Q[f0 + t] * Dkl);" % cd)
     o.append("                    R[%d + NCD + t] = qd;" % KREC0)
     o.append("                    beta = fmax(beta, qd);")
+    if rys:
+        # a component whose density weight is zero adds nothing, masked or not
+        o.append("                    qmin = fmin(qmin, Dkl != 0.0 ? qd : qmin);")
     o.append("                }")
+    if rys:
+        o.append("                R[%d] = qmin;" % (rec - 1))
     o.append("                R[0] = beta;")
     o.append("            }")
     o.append("        }")
@@ -585,15 +743,51 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
             lines += [ind + x for x in _dag_lines(dag)]
         return lines
 
+    def jrys(tyq, ind):
+        """The quartet by Rys quadrature, as the exchange kernels' krys."""
+        TAU = (lambda t: "tau[%d * TILE_SIZE_J + lane]" % t) if jlds else (lambda t: "tau[%d]" % t)
+        ACC = (lambda t: "lacc[%d * TILE_SIZE_J + lane]" % t) if jlds else (lambda t: "acc[%d]" % t)
+        lines = rys_prologue(L, ind=ind)
+        lines.append(ind + "const bool whole = __all(!live || R[%d] > taumax);" % (rec - 1))
+        for isl, group in enumerate(jsl):
+            lines.append(ind + "{")
+            lines += rys_pass(la, lb, lc, ld, group, "g%d_" % isl, ind + "    ")
+            for ic, idd in group:
+                tcd = ic * nd + idd
+                lines.append(ind + "    const double Dp%d = R[%d], Qd%d = R[%d];" % (tcd, KREC0 + tcd, tcd, KREC0 + ncd + tcd))
+            for masked in (False, True):
+                lines.append(ind + ("    } else if (live) {" if masked else "    if (whole && live) {"))
+                for tab in range(nab):
+                    terms = []
+                    for ic, idd in group:
+                        tcd = ic * nd + idd
+                        term = "X%d_%d * Dp%d" % (tab, tcd, tcd)
+                        terms.append("((Qd%d > %s) ? %s : 0.0)" % (tcd, TAU(tab), term) if masked else term)
+                    lines.append(ind + "        %s += %s;" % (ACC(tab), " + ".join(terms)))
+            lines += [ind + "    }", ind + "}"]
+        return lines
+
     # J keeps its passes inside one ket loop (the bra-side state is small);
     # measured faster than one loop per pass
     # the FP32 loop of a mixed kernel may run fewer passes (half-size values)
     jsl32 = plan_slices_f32(la, lb, lc, ld, "J") if mixed else jsl
-    o += ket_loops("        ", "active", "qmax * R[0] * (1.0 + 1e-13) <= thr", "qmax * R[0]", KET_HEADER,
-                   lambda ty, ind: jbody(ty, ind, jsl if ty == "double" else jsl32), mixed, "lo_mode",
-                   count=mixed or batched)
+    jscreen = "qmax * R[0] * (1.0 + 1e-13) <= thr"
+    if rys:
+        o += rys_ket_loop("        ", jscreen, KET_HEADER, jrys, count=batched)
+    else:
+        o += ket_loops("        ", "active", jscreen, "qmax * R[0]", KET_HEADER,
+                       lambda ty, ind: jbody(ty, ind, jsl if ty == "double" else jsl32), mixed, "lo_mode",
+                       count=mixed or batched, pack=pack)
     o.append("    }")
-    o.append("    if (own) {")
+    if pack:
+        # the lane groups' sums of a block, added in a fixed order
+        o.append("    #pragma unroll")
+        o.append("    for (int t = 0; t < NAB; ++t) {")
+        o.append("        double v = %s;" % ("lacc[t * TILE_SIZE_J + lane]" if jlds else "acc[t]"))
+        o.append("        for (uint32_t off = 1u << wsh; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);")
+        o.append("        %s = v;" % ("lacc[t * TILE_SIZE_J + lane]" if jlds else "acc[t]"))
+        o.append("    }")
+    o.append("    if (own%s) {" % (" && slot == 0" if pack else ""))
     o.append("        const uint32_t e0 = bb * NAB;")
     o.append("        #pragma unroll")
     o.append("        for (int t = 0; t < NAB; ++t) {")
@@ -698,7 +892,8 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
 # K kernel
 # --------------------------------------------------------------------------
 
-def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", lds_boys=False, wpg=1, kpairs=False):
+def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", lds_boys=False, wpg=1, kpairs=False,
+           rys=None, pack=False):
     """Source of computeExchangeFock{CLS} (or its _mixed / _batched variants) and
     its launcher.  The batched variant is persistent over a list of (i,k) blocks
     of lists that concatenate many molecules; per block, blk_mol gives the
@@ -711,7 +906,15 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     64 lanes of a wave (64 partners j, one ket partner l) read 64 rows; "lj"
     reads D[l][j], so the wave reads one row of D at 64 columns.  The two agree
     for a symmetric density (every SCF density; the host symmetrises it
-    exactly), and the faster one per class is a measured choice."""
+    exactly), and the faster one per class is a measured choice.
+
+    ``rys`` ({"maxx", "tau", "waves"}, FP64 only): evaluate the quartet by Rys
+    quadrature (rysdag) in passes of at most ``maxx`` component sums; "tau"
+    says where the per-lane thresholds and S_ab are kept ("reg" or "lds"),
+    "waves" the wavefronts per SIMD the registers are allotted for.  ``pack``:
+    a tile of few partners J shares its lanes out among several ket records
+    (pack_decls; Rys kernels always do)."""
+    pack = pack or rys is not None
     a, b, c, d = cls
     la, lb, lc, ld = LV[a], LV[b], LV[c], LV[d]
     na, nb, nc, nd = NC[a], NC[b], NC[c], NC[d]
@@ -722,6 +925,10 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     rec += rec % 2
     kslices = plan_slices(la, lb, lc, ld, "Kheavy")
     heavy = len(kslices) > 1
+    if rys:
+        assert not mixed, "Rys bodies are for the FP64 kernels"
+        heavy, layout, lds_boys = False, "reg", False
+        kslices = rys_groups(nab, nc, nd, rys["maxx"])
     if heavy and kpairs:
         # one pass per ket component pair (ic, id): the recursion is recomputed
         # per pair, and only one pair's intermediates are live at a time
@@ -735,7 +942,8 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     ty = "double"
     o = []
     assert not (heavy and wpg > 1), "the heavy layouts keep one wavefront per workgroup"
-    o.append("__global__ void __launch_bounds__(%s)" % ("TILE_SIZE_K" if wpg == 1 else str(64 * wpg)))
+    o.append("__global__ void __launch_bounds__(%s%s)" % ("TILE_SIZE_K" if wpg == 1 else str(64 * wpg),
+                                                         ", %d" % rys["waves"] if rys and rys.get("waves") else ""))
     o.append("%s(%s)" % (name, ",\n    ".join(sig)))
     o.append("{")
     o.append("    constexpr int NA = %d, NB = %d, NC = %d, ND = %d, NAC = %d, NAB = %d, NCD = %d;" % (na, nb, nc, nd, nac, nab, ncd))
@@ -756,10 +964,12 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     #          they fit beside the thresholds, S_ab and an 8-record ket tile in one
     #          wave's LDS share, and b-major digestion with each b's density row
     #          loaded just before its block.
+    lds_tau = heavy or (rys is not None and rys["tau"] == "lds")
     lds_layout = heavy and layout == "lds"
     lacc = lds_layout and (16 * nab + 8 * nac) * 64 + 8 * ket_record_bytes("K", cls) <= LDS_PER_WAVE_FULL_REGS
-    if heavy:
+    if lds_tau:
         # per-lane thresholds and S_ab live in LDS ([component][lane]) to free registers
+        assert wpg == 1
         o.append("    __shared__ double ltau[NAB * TILE_SIZE_K], lSab[NAB * TILE_SIZE_K];")
     if lacc:
         # per-lane K accumulators in LDS ([component][lane]); a pass keeps its
@@ -771,6 +981,8 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         o.append("    uint32_t* ket_cg = ket_cg_all + wave * (KT * ND);")
     if lds_boys:
         o += lds_boys_setup(L)
+    if rys:
+        o += rys_decl(L, wpg)
     if mixed or batched:
         o += count_decl()
     if batched:
@@ -816,13 +1028,20 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         o.append("    double acc[NAC];")
         o.append("    #pragma unroll")
         o.append("    for (int t = 0; t < NAC; ++t) acc[t] = 0.0;")
-    o.append("    for (uint32_t jc = 0; jc < nJ; jc += TILE_SIZE_K) {")
-    o.append("        const uint32_t jp = jc + lane;")
+    if pack:
+        o.append("    for (uint32_t jc = 0, jw; jc < nJ; jc += jw) {")
+        o.append("        const uint32_t left = nJ - jc;")
+        o += pack_decls("        ", "left")
+        o.append("        jw = 1u << wsh;")
+        o.append("        const uint32_t jp = jc + jl;")
+    else:
+        o.append("    for (uint32_t jc = 0; jc < nJ; jc += TILE_SIZE_K) {")
+        o.append("        const uint32_t jp = jc + lane;")
     o.append("        bool active = jp < nJ;")
     o.append("        double zeta = 1.0, sq_zeta = 1.0, inv_S1 = 1.0, P_x = 0.0, P_y = 0.0, P_z = 0.0;")
     o.append("        double PA_x = 0.0, PA_y = 0.0, PA_z = 0.0, AB_x = 0.0, AB_y = 0.0, AB_z = 0.0;")
-    o.append("        double qij = 0.0;")
-    if heavy:
+    o.append("        double qij = 0.0%s;" % (", taumax = 0.0" if rys else ""))
+    if lds_tau:
         o.append("        double* tau = ltau;")
         o.append("        double* Sab = lSab;")
         o.append("        #pragma unroll")
@@ -850,7 +1069,10 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                    const uint32_t pos = displ_i[ca] + jp * NB + cb;")
     o.append("                    const double q = fabs(Q_K_%s[pos]);" % ab)
     o.append("                    qij = fmax(qij, q);")
-    if heavy:
+    if rys:
+        # 0/0 (a zero bound at a zero threshold) passes nothing, like infinity
+        o.append("                    if (pair_data_K_%s[pos] != 0.0) taumax = fmax(taumax, thr_eff / q >= 0.0 ? thr_eff / q : __builtin_inf());" % ab)
+    if lds_tau:
         o.append("                    tau[(ca * NB + cb) * TILE_SIZE_K + lane] = thr_eff / q;")
         o.append("                    Sab[(ca * NB + cb) * TILE_SIZE_K + lane] = pair_data_K_%s[pos];" % ab)
     else:
@@ -885,7 +1107,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                    R[3] = (ak * C_x + al * D_x) * iet; R[4] = (ak * C_y + al * D_y) * iet; R[5] = (ak * C_z + al * D_z) * iet;")
     o.append("                    R[6] = (al * iet) * (D_x - C_x); R[7] = (al * iet) * (D_y - C_y); R[8] = (al * iet) * (D_z - C_z);")
     o.append("                    R[9] = C_x - D_x; R[10] = C_y - D_y; R[11] = C_z - D_z;")
-    o.append("                    double qk = 0.0;")
+    o.append("                    double qk = 0.0%s;" % (", qmin = __builtin_inf()" if rys else ""))
     o.append("                    #pragma unroll")
     o.append("                    for (int cc = 0; cc < NC; ++cc) {")
     o.append("                        #pragma unroll")
@@ -893,11 +1115,16 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                            const uint32_t pos = displ_k[cc] + lp * ND + cdd;")
     o.append("                            const double q = fabs(Q_K_%s[pos]);" % cd)
     o.append("                            qk = fmax(qk, q);")
+    if rys:
+        # a component whose factor is zero adds nothing, masked or not
+        o.append("                            if (pair_data_K_%s[pos] != 0.0) qmin = fmin(qmin, q);" % cd)
     o.append("                            R[%d + cc * ND + cdd] = pair_data_K_%s[pos];" % (KREC0, cd))
     o.append("                            R[%d + NCD + cc * ND + cdd] = q;" % KREC0)
     o.append("                        }")
     o.append("                    }")
     o.append("                    R[0] = qk;")
+    if rys:
+        o.append("                    R[%d] = qmin;" % (rec - 1))
     o.append("                    #pragma unroll")
     o.append("                    for (int cdd = 0; cdd < ND; ++cdd) {")
     o.append("                        const uint32_t ll = D_inds_K_%s[displ_k[0] + lp * ND + cdd];" % cd)
@@ -985,6 +1212,42 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
             lines += [ind + x for x in _dag_lines(dag)]
         return lines
 
+    def krys(tyq, ind):
+        """The quartet by Rys quadrature.  Per pass: the density gathers, the
+        component sums (the point loop hides the gathers), then the digestion
+        acc[a,c] += Sc_cd sum_b (S_ab D_bd) X -- without masks when every
+        component of every live lane's quartet passes the screen (one uniform
+        test per quartet)."""
+        TAU = (lambda t: "tau[%d * TILE_SIZE_K + lane]" % t) if lds_tau else (lambda t: "tau[%d]" % t)
+        SAB = (lambda t: "Sab[%d * TILE_SIZE_K + lane]" % t) if lds_tau else (lambda t: "Sab[%d]" % t)
+        lines = rys_prologue(L, omega=True, ind=ind)
+        lines.append(ind + "const bool whole = __all(!live || R[%d] > taumax);" % (rec - 1))
+        for isl, group in enumerate(kslices):
+            idds = sorted({d_ for _, d_ in group})
+            lines.append(ind + "{")
+            for idd in idds:
+                for ib in range(nb):
+                    lines.append(ind + "    const double Dj%d_%d = %s;" % (ib, idd, dread("cgJ[%d]" % ib, idd)))
+            lines += rys_pass(la, lb, lc, ld, group, "g%d_" % isl, ind + "    ")
+            for idd in idds:
+                for tab in range(nab):
+                    lines.append(ind + "    const double v%d_%d = %s * Dj%d_%d;" % (tab, idd, SAB(tab), tab % nb, idd))
+            for masked in (False, True):
+                lines.append(ind + ("    } else if (live) {" if masked else "    if (whole && live) {"))
+                for ic, idd in group:
+                    tcd = ic * nd + idd
+                    lines.append(ind + "        const double Sc%d = R[%d]%s;"
+                                 % (tcd, KREC0 + tcd, ", Qk%d = R[%d]" % (tcd, KREC0 + ncd + tcd) if masked else ""))
+                    for ia in range(na):
+                        terms = []
+                        for ib in range(nb):
+                            tab = ia * nb + ib
+                            term = "v%d_%d * X%d_%d" % (tab, idd, tab, tcd)
+                            terms.append("((Qk%d > %s) ? %s : 0.0)" % (tcd, TAU(tab), term) if masked else term)
+                        lines.append(ind + "        acc[%d] += Sc%d * (%s);" % (ia * nc + ic, tcd, " + ".join(terms)))
+            lines += [ind + "    }", ind + "}"]
+        return lines
+
     kscreen = "qij * R[0] * maxD * (1.0 + 1e-13) <= thr"
     kbound = "qij * R[0] * maxD"
     def pacc_io(group, store):
@@ -1000,7 +1263,9 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         return out
 
     kslices32 = plan_slices_f32(la, lb, lc, ld, "Kheavy") if mixed else kslices
-    if heavy and len(kslices32) == len(kslices):
+    if rys:
+        o += rys_ket_loop("            ", kscreen, KET_HEADER, krys, count=batched)
+    elif heavy and len(kslices32) == len(kslices):
         # heavy classes: one loop over the tile per pass of ket-first-index
         # components, so that only one pass's recursion is live at a time; the
         # screening sequence is the same in every pass, so each pass stops at
@@ -1016,7 +1281,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
             o += pacc_io(group, False)
             o += ket_loops("            ", "act%d" % isl, kscreen, kbound, KET_HEADER,
                            lambda ty, ind, g=group: kbody(ty, ind, [g]), mixed, "lo%d" % isl,
-                           count=(mixed or batched) and isl == 0)
+                           count=(mixed or batched) and isl == 0, pack=pack)
             o += pacc_io(group, True)
             o.append("            act_end = act%d;" % isl)
             if mixed:
@@ -1030,20 +1295,21 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         # FP64 passes (one loop each) run up to the first record where the
         # whole wavefront is below fp32_threshold (the same record in every
         # pass: identical screening), then the FP32 passes run from there
+        sv = "sb" if pack else "s"
         o.append("            uint32_t s_sw = 0;")
         o.append("            bool act_sw = active, lo_sw = lo_mode;")
         for isl, group in enumerate(kslices):
             o.append("            {")
             o.append("            bool act%d = active, lo%d = lo_mode;" % (isl, isl))
             o += pacc_io(group, False)
-            o.append("            uint32_t s = 0;")
+            o.append("            uint32_t %s = 0;" % sv)
             o.append("            if (!lo%d) {" % isl)
             o += ["    " + x for x in ket_loop("            ", "act%d" % isl, kscreen, kbound, KET_HEADER,
                                              lambda ty, ind, g=group: kbody(ty, ind, [g]), "double", True,
-                                             "lo%d" % isl, count=isl == 0)]
+                                             "lo%d" % isl, count=isl == 0, pack=pack)]
             o.append("            }")
             o += pacc_io(group, True)
-            o.append("            s_sw = s; act_sw = act%d; lo_sw = lo%d;" % (isl, isl))
+            o.append("            s_sw = %s; act_sw = act%d; lo_sw = lo%d;" % (sv, isl, isl))
             o.append("            }")
         o.append("            bool act_end = act_sw;")
         o.append("            if (lo_sw) {")
@@ -1051,9 +1317,9 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
             o.append("            {")
             o.append("            bool actf%d = act_sw;" % isl)
             o += pacc_io(group, False)
-            o.append("            uint32_t s = s_sw;")
+            o.append("            uint32_t %s = s_sw;" % sv)
             o += ket_loop("            ", "actf%d" % isl, kscreen, kbound, KET_HEADER,
-                          lambda ty, ind, g=group: kbody(ty, ind, [g]), "float", False, "lo_sw", count=isl == 0)
+                          lambda ty, ind, g=group: kbody(ty, ind, [g]), "float", False, "lo_sw", count=isl == 0, pack=pack)
             o += pacc_io(group, True)
             o.append("            act_end = actf%d;" % isl)
             o.append("            }")
@@ -1063,7 +1329,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     else:
         o += ket_loops("            ", "active", kscreen, kbound, KET_HEADER,
                        lambda ty, ind: kbody(ty, ind, [list(range(nc))]), mixed, "lo_mode",
-                       count=mixed or batched)
+                       count=mixed or batched, pack=pack)
     o.append("        }")
     o.append("    }")
     o.append("    #pragma unroll")

@@ -33,7 +33,8 @@ pass or in one pass per ket-first-index component, a per-class choice
 from __future__ import annotations
 
 from .emit import (KET_HEADER, KET_TILE, KREC0, LV, NC, _argnames, _dag_lines, _strip_restrict,
-                   j_signature, k_signature, ket_loops, launder, quartet_prologue)
+                   j_signature, k_signature, ket_loops, launder, pack_decls, pack_decls1, quartet_prologue, rys_decl, rys_grad_pass,
+                   rys_groups, rys_ket_loop, rys_prologue)
 from .osdag import QuartetDAG, add, tri
 
 AXES = "xyz"
@@ -98,7 +99,13 @@ def ket_tile(rec_doubles, extra_bytes=0):
     return kt
 
 
-def emit_jgrad(cls, passes="one"):
+def rys_ket_tile(nab, ncd):
+    """Ket tile of a Rys kernel: 16 records, 8 where a (dd| or |dd) class's
+    records or per-lane thresholds take most of a wavefront's 40 KB of LDS."""
+    return 8 if max(nab, ncd) >= 36 else 16
+
+
+def emit_jgrad(cls, passes="one", rys=None):
     """Source of computeCoulombGradient{CLS} and its launcher.
 
     Kernel: blockDim 64, gridDim (ceil(bra blocks / 64), ket chunks); chunk y
@@ -116,17 +123,21 @@ def emit_jgrad(cls, passes="one"):
     rec += rec % 2
     name = "computeCoulombGradient" + cls.upper()
     sig = jg_signature(cls)
-    groups = grad_groups(la, lb, lc, ld, passes)
-    o = ["__global__ void __launch_bounds__(64)",
+    groups = rys_groups(nab, nc, nd, rys["maxx"]) if rys else grad_groups(la, lb, lc, ld, passes)
+    lds = rys is not None and rys["tau"] == "lds"
+    at = "%s * 64 + lane" if lds else "%s"
+    o = ["__global__ void __launch_bounds__(64%s)" % (", %d" % rys["waves"] if rys and rys.get("waves") else ""),
          "%s(%s)" % (name, ",\n    ".join(sig)),
          "{",
          "    constexpr int NA = %d, NB = %d, NC = %d, ND = %d, NAB = %d, NCD = %d;" % (na, nb, nc, nd, nab, ncd),
-         "    constexpr int KT = %d, REC = %d;" % (ket_tile(rec), rec),
+         "    constexpr int KT = %d, REC = %d;" % (rys_ket_tile(nab, ncd) if rys else ket_tile(rec), rec),
          "    __shared__ double ket[KT * REC];",
          "    const uint32_t lane = threadIdx.x;",
          "    const uint32_t nbra = %s_prim_pair_count_local / NAB;" % ab,
          "    const uint32_t nket = %s_prim_pair_count / NCD;" % cd,
-         "    const uint32_t bb = blockIdx.x * 64 + lane;",
+         "    const uint32_t left = nbra - blockIdx.x * 64;",
+         "\n".join(pack_decls1("    ", "left")),
+         "    const uint32_t bb = blockIdx.x * 64 + jl;",
          "    const uint32_t chunk = (nket + gridDim.y - 1) / gridDim.y;",
          "    const uint32_t k_begin = blockIdx.y * chunk;",
          "    const uint32_t k_end = (k_begin + chunk < nket) ? (k_begin + chunk) : nket;",
@@ -136,11 +147,12 @@ def emit_jgrad(cls, passes="one"):
          "    double zeta = 1.0, sq_zeta = 1.0, inv_S1 = 1.0, P_x = 0.0, P_y = 0.0, P_z = 0.0;",
          "    double PA_x = 0.0, PA_y = 0.0, PA_z = 0.0, AB_x = 0.0, AB_y = 0.0, AB_z = 0.0;",
          "    double two_ai = 0.0, two_aj = 0.0, qmax = 0.0;",
-         "    double tau[NAB], wab[NAB];",
+         "    __shared__ double tau[NAB * 64], wab[NAB * 64];" if lds else "    double tau[NAB], wab[NAB];",
          "    double gacc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};",
          "    #pragma unroll",
-         "    for (int t = 0; t < NAB; ++t) { tau[t] = 0.0; wab[t] = 0.0; }",
-         "    if (active) {",
+         "    for (int t = 0; t < NAB; ++t) { tau[%s] = 0.0; wab[%s] = 0.0; }" % (at % "t", at % "t")]
+    o += rys_decl(L) if rys else []
+    o += ["    if (active) {",
          "        const uint32_t e0 = bb * NAB;",
          "        const uint32_t I = %s_first_inds_local[e0] / NA;" % ab,
          "        const uint32_t J = %s_second_inds_local[e0] / NB;" % ab,
@@ -157,12 +169,12 @@ def emit_jgrad(cls, passes="one"):
          "        for (int t = 0; t < NAB; ++t) {",
          "            const double q = fabs(%s_mat_Q_local[e0 + t]);" % ab,
          "            qmax = fmax(qmax, q);",
-         "            tau[t] = thr / q;"]
+         "            tau[%s] = thr / q;" % (at % "t")]
     if a == b:
         o.append("            const double w = (%s_first_inds_local[e0 + t] != %s_second_inds_local[e0 + t]) ? 2.0 : 1.0;" % (ab, ab))
     else:
         o.append("            const double w = 2.0;")
-    o += ["            wab[t] = %s_pair_data_local[e0 + t] * %s_mat_D_local[e0 + t] * w;" % (ab, ab),
+    o += ["            wab[%s] = %s_pair_data_local[e0 + t] * %s_mat_D_local[e0 + t] * w;" % (at % "t", ab, ab),
           "        }",
           "    }",
           "    for (uint32_t t0 = k_begin; t0 < k_end; t0 += KT) {",
@@ -203,6 +215,21 @@ def emit_jgrad(cls, passes="one"):
           "        __syncthreads();",
           "        const uint32_t nt = (k_end - t0 < (uint32_t)KT) ? (k_end - t0) : (uint32_t)KT;"]
 
+    def rys_body(tyq, ind):
+        """Per pass: the masked component weights, then the point loop."""
+        lines = rys_prologue(L, ind=ind)
+        for isl, group in enumerate(groups):
+            lines.append(ind + "{")
+            for ic, idd in group:
+                tcd = ic * nd + idd
+                lines.append(ind + "    const double Dp%d = R[%d], Qd%d = R[%d];" % (tcd, KREC0 + tcd, tcd, KREC0 + ncd + tcd))
+                for tab in range(nab):
+                    lines.append(ind + "    const double W%d_%d = (live && Qd%d > tau[%s]) ? wab[%s] * Dp%d : 0.0;"
+                                 % (tab, tcd, tcd, at % tab, at % tab, tcd))
+            lines += rys_grad_pass(la, lb, lc, ld, group, [(0, "two_ai", 0), (1, "two_aj", 3)], "g%d_" % isl, ind + "    ")
+            lines.append(ind + "}")
+        return lines
+
     def body(tyq, ind):
         lines = quartet_prologue(L, ind=ind)
         for isl, group in enumerate(groups):
@@ -228,10 +255,13 @@ def emit_jgrad(cls, passes="one"):
             lines += [ind + x for x in _dag_lines(dag)]
         return lines
 
-    o += ket_loops("        ", "active", "qmax * R[0] * (1.0 + 1e-13) <= thr", "qmax * R[0]", KET_HEADER,
-                   body, False, "lo_mode", count=False)
+    if rys:
+        o += rys_ket_loop("        ", "qmax * R[0] * (1.0 + 1e-13) <= thr", KET_HEADER, rys_body)
+    else:
+        o += ket_loops("        ", "active", "qmax * R[0] * (1.0 + 1e-13) <= thr", "qmax * R[0]", KET_HEADER, body, False, "lo_mode", count=False, pack=True)
     o += ["    }",
-          "    if (own) {",
+          "    for (int g = 0; g < 6; ++g) for (uint32_t off = 1u << wsh; off < 64; off <<= 1) gacc[g] += __shfl_xor(gacc[g], off, 64);",
+          "    if (own && slot == 0) {",
           "        double* row = grad_%s + ((size_t)blockIdx.y * nbra + bb) * 6;" % ab,
           "        #pragma unroll",
           "        for (int g = 0; g < 6; ++g) row[g] = gacc[g];",
@@ -268,15 +298,16 @@ def emit_jgrad(cls, passes="one"):
     return "\n".join(o) + "\n"
 
 
-def emit_kgrad(cls, passes="one", split=False):
+def emit_kgrad(cls, passes="one", rys=None, centres=False):
     """Source of computeExchangeGradient{CLS} and its launcher.
 
     Kernel: blockDim 64, gridDim = (i,k) blocks; lane 0 adds the wavefront's
     six sums to grad[blk * 6 + 0..5] (A-centre x, y, z, then C-centre x, y, z);
-    one wavefront per block, so one writer per row.  With ``split`` the
-    A-centre and C-centre parts are two kernels (``_A``, ``_C``), each with
-    one raised recursion (a+1 on the bra, or c+1 on the ket) instead of both,
-    which the launcher runs one after the other."""
+    one wavefront per block, so one writer per row.  With ``centres`` the
+    source also holds the kernels of the A-centre part (``_A``, columns 0..2)
+    and of the C-centre part (``_C``, columns 3..5) alone, for code that
+    launches kernels directly; the launcher runs the one for both, which
+    shares the quadrature points and the component sums."""
     a, b, c, d = cls
     la, lb, lc, ld = LV[a], LV[b], LV[c], LV[d]
     na, nb, nc, nd = NC[a], NC[b], NC[c], NC[d]
@@ -287,10 +318,13 @@ def emit_kgrad(cls, passes="one", split=False):
     rec += rec % 2
     name = "computeExchangeGradient" + cls.upper()
     sig = kg_signature(cls)
-    groups = grad_groups(la, lb, lc, ld, passes)
-    kt = ket_tile(rec, 4 * nd)
+    groups = rys_groups(nab, nc, nd, rys["maxx"]) if rys else grad_groups(la, lb, lc, ld, passes)
+    kt = rys_ket_tile(nab, ncd) if rys else ket_tile(rec, 4 * nd)
+    lds = rys is not None and rys["tau"] == "lds"
+    at = "%s * 64 + lane" if lds else "%s"
+
     def kernel(kname, cents):
-        o = ["__global__ void __launch_bounds__(64)",
+        o = ["__global__ void __launch_bounds__(64%s)" % (", %d" % rys["waves"] if rys and rys.get("waves") else ""),
              "%s(%s)" % (kname, ",\n    ".join(sig)),
              "{",
              "    constexpr int NA = %d, NB = %d, NC = %d, ND = %d, NAC = %d, NAB = %d, NCD = %d;" % (na, nb, nc, nd, nac, nab, ncd),
@@ -330,16 +364,23 @@ def emit_kgrad(cls, passes="one", split=False):
              "    for (int t = 0; t < NC; ++t) displ_k[t] = pair_displs_K_%s[K * NC + t];" % cd,
              "    const uint32_t nJ = pair_counts_K_%s[I * NA] / NB;" % ab,
              "    const uint32_t nL = pair_counts_K_%s[K * NC] / ND;" % cd,
-             "    double gacc[%d] = {%s};" % (3 * len(cents), ", ".join(["0.0"] * (3 * len(cents)))),
-             "    for (uint32_t jc = 0; jc < nJ; jc += 64) {",
-             "        const uint32_t jp = jc + lane;",
+             "    double gacc[%d] = {%s};" % (3 * len(cents), ", ".join(["0.0"] * (3 * len(cents))))]
+        if lds:
+            o.append("    __shared__ double tau[NAB * 64], Sab[NAB * 64];")
+        if rys:
+            o += rys_decl(L)
+        o += ["    for (uint32_t jc = 0, jw; jc < nJ; jc += jw) {",
+              "        const uint32_t left = nJ - jc;"] + pack_decls("        ", "left") + [
+              "        jw = 1u << wsh;",
+              "        const uint32_t jp = jc + jl;"]
+        o += [
              "        bool active = jp < nJ;",
              "        double zeta = 1.0, sq_zeta = 1.0, inv_S1 = 1.0, P_x = 0.0, P_y = 0.0, P_z = 0.0;",
              "        double PA_x = 0.0, PA_y = 0.0, PA_z = 0.0, AB_x = 0.0, AB_y = 0.0, AB_z = 0.0;",
              "        double qij = 0.0;",
-             "        double tau[NAB], Sab[NAB];",
+             "" if lds else "        double tau[NAB], Sab[NAB];",
              "        #pragma unroll",
-             "        for (int t = 0; t < NAB; ++t) { tau[t] = 0.0; Sab[t] = 0.0; }",
+             "        for (int t = 0; t < NAB; ++t) { tau[%s] = 0.0; Sab[%s] = 0.0; }" % (at % "t", at % "t"),
              "        uint32_t cgJ[NB];",
              "        #pragma unroll",
              "        for (int t = 0; t < NB; ++t) cgJ[t] = 0;",
@@ -359,8 +400,8 @@ def emit_kgrad(cls, passes="one", split=False):
              "                    const uint32_t pos = displ_i[ca] + jp * NB + cb;",
              "                    const double q = fabs(Q_K_%s[pos]);" % ab,
              "                    qij = fmax(qij, q);",
-             "                    tau[ca * NB + cb] = thr_eff / q;",
-             "                    Sab[ca * NB + cb] = pair_data_K_%s[pos];" % ab,
+             "                    tau[%s] = thr_eff / q;" % (at % "(ca * NB + cb)"),
+             "                    Sab[%s] = pair_data_K_%s[pos];" % (at % "(ca * NB + cb)", ab),
              "                }",
              "            }",
              "            #pragma unroll",
@@ -414,6 +455,30 @@ def emit_kgrad(cls, passes="one", split=False):
               "            __syncthreads();",
               "            const uint32_t nt = (nL - t0 < (uint32_t)KT) ? (nL - t0) : (uint32_t)KT;"]
 
+        def rys_body(tyq, ind):
+            """Per pass: the masked component weights, then the point loop."""
+            lines = rys_prologue(L, omega=True, ind=ind)
+            for isl, group in enumerate(groups):
+                idds = sorted({d_ for _, d_ in group})
+                lines.append(ind + "{")
+                for idd in idds:
+                    for ib in range(nb):
+                        lines.append(ind + "    const double Dj%d_%d = Dm[(size_t)ket_cg[s * ND + %d] * nao + cgJ[%d]];" % (ib, idd, idd, ib))
+                    for tab in range(nab):
+                        lines.append(ind + "    const double v%d_%d = Sab[%s] * Dj%d_%d;" % (tab, idd, at % tab, tab % nb, idd))
+                for ic, idd in group:
+                    tcd = ic * nd + idd
+                    lines.append(ind + "    const double Sc%d = R[%d], Qk%d = R[%d];" % (tcd, KREC0 + tcd, tcd, KREC0 + ncd + tcd))
+                    for ia in range(na):
+                        lines.append(ind + "    const double u%d_%d = Dac[%d] * Sc%d;" % (ia, tcd, ia * nc + ic, tcd))
+                    for tab in range(nab):
+                        lines.append(ind + "    const double W%d_%d = (live && Qk%d > tau[%s]) ? u%d_%d * v%d_%d : 0.0;"
+                                     % (tab, tcd, tcd, at % tab, tab // nb, tcd, tab, idd))
+                lines += rys_grad_pass(la, lb, lc, ld, group, [(p, two, 3 * k) for k, (p, two, _) in enumerate(cents)],
+                                       "g%d_" % isl, ind + "    ")
+                lines.append(ind + "}")
+            return lines
+
         def body(tyq, ind):
             lines = quartet_prologue(L, omega=True, ind=ind)
             for ibb in range(nb):
@@ -444,8 +509,11 @@ def emit_kgrad(cls, passes="one", split=False):
                 lines += [ind + x for x in _dag_lines(dag)]
             return lines
 
-        o += ket_loops("            ", "active", "qij * R[0] * maxD * (1.0 + 1e-13) <= thr", "qij * R[0] * maxD",
-                       KET_HEADER, body, False, "lo_mode", count=False)
+        if rys:
+            o += rys_ket_loop("            ", "qij * R[0] * maxD * (1.0 + 1e-13) <= thr", KET_HEADER, rys_body)
+        else:
+            o += ket_loops("            ", "active", "qij * R[0] * maxD * (1.0 + 1e-13) <= thr", "qij * R[0] * maxD",
+                           KET_HEADER, body, False, "lo_mode", count=False, pack=True)
         o += ["        }",
               "    }",
               "    #pragma unroll",
@@ -461,7 +529,7 @@ def emit_kgrad(cls, passes="one", split=False):
 
     # (position, 2 x exponent, first output column) of the centres a kernel covers
     both = [(0, "two_ai", 0), (2, "two_ak", 3)]
-    parts = [(name, both)] if not split else [(name + "_A", both[:1]), (name + "_C", both[1:])]
+    parts = [(name, both)] + ([(name + "_A", both[:1]), (name + "_C", both[1:])] if centres else [])
     o = []
     for kname, cents in parts:
         o += kernel(kname, cents)
@@ -483,12 +551,7 @@ def emit_kgrad(cls, passes="one", split=False):
                  % (lc, ld, c, cd, cd, cd, cd))
     o += ["        if (rc != 0) return rc;",
           "    }"]
-    for kn, _ in parts:
-        o += ["    hipLaunchKernelGGL(%s, dim3(nblk), dim3(64), 0, (hipStream_t)stream, %s);" % (kn, ", ".join(args)),
-              "    {",
-              "        const int rc = (int)hipGetLastError();",
-              "        if (rc != 0) return rc;",
-              "    }"]
-    o += ["    return VLXMI_OK;",
+    o += ["    hipLaunchKernelGGL(%s, dim3(nblk), dim3(64), 0, (hipStream_t)stream, %s);" % (name, ", ".join(args)),
+          "    return (int)hipGetLastError();",
           "}"]
     return "\n".join(o) + "\n"
