@@ -84,7 +84,7 @@ template <int L>
 __global__ void boys_coarse_probe_kernel(const double* __restrict__ T, uint32_t n,
                                          const double* __restrict__ table, double* __restrict__ out)
 {
-    __shared__ double lt[VLX_BOYS_CROWS * VLX_BOYS_CTERMS];
+    __shared__ double lt[VLX_BOYS_LROWS * VLX_BOYS_LCOLS];
     vlxmi::boys_lds_fill<L>(table, lt);
     __syncthreads();
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -95,8 +95,8 @@ __global__ void boys_coarse_probe_kernel(const double* __restrict__ T, uint32_t 
     for (int m = 0; m <= L; ++m) out[(size_t)t * (L + 1) + m] = F[m];
 }
 
-// As vlxmi_boys_eval, through the coarse rows copied to LDS (the evaluation
-// some light-class kernels use); L = 0..4.
+// As vlxmi_boys_eval, through the rows kept in LDS (the evaluation the
+// light-class kernels use); L = 0..4.
 extern "C" int vlxmi_boys_eval_coarse(const double* T, uint32_t n, uint32_t L, const double* table, double* out,
                                       void* stream)
 {

@@ -28,11 +28,10 @@
 // single-precision hardware exponential is accurate enough for it.
 //
 // Coarse rows (after the fine table, VLX_BOYS_CROWS rows of VLX_BOYS_NCOL
-// doubles): F_0..F_15 at T_k = k * VLX_BOYS_CDT.  Kernels of a few light
-// classes copy the 12 columns F_L..F_{L+11} of these rows, scaled by 1/j!, into
-// LDS once per workgroup (9.7 KB) and evaluate F_L by a 12-term Taylor expansion
-// about the nearest coarse point, |T - T_k| <= 0.2, remainder below
-// 0.2^12 / 12! = 8.6e-18 (relative to F_L): no global gather per quartet.
+// doubles): F_0..F_15 at T_k = k * VLX_BOYS_CDT; kept in the table's layout, no
+// kernel reads them.  Kernels of the light classes make their own rows in LDS
+// from every tenth fine row, once per workgroup (boys_lds_fill), and evaluate
+// F_L from there: no global gather per quartet.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -64,6 +63,8 @@ extern "C" int vlxmi_ket_split_reduce(const double* part, uint32_t nsplit, uint3
 #define VLX_BOYS_CDT 0.4
 #define VLX_BOYS_INV_CDT 2.5
 #define VLX_BOYS_CTERMS 12
+#define VLX_BOYS_LROWS 200
+#define VLX_BOYS_LCOLS 10
 #define VLX_BOYS_COARSE_OFF (VLX_BOYS_NROW * VLX_BOYS_NCOL)
 
 #define MATH_CONST_PI 3.14159265358979323846
@@ -87,25 +88,21 @@ __device__ __forceinline__ void wave_sync()
 
 // 1/x and 1/sqrt(x) for positive, normal x well inside the double range (the
 // Gaussian exponent sums and Boys arguments these are used on): the hardware
-// estimate refined by two Newton steps, each of which squares the relative
-// error, so the result is within a few ulp; no denormal/overflow scaling.
+// estimate (relative error below 2^-22) refined by one third-order step, which
+// cubes that error, so the result is within a few ulp; no denormal/overflow
+// scaling.
 __device__ __forceinline__ double rcp_nr(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 __device__ __forceinline__ double rsq_nr(double x)
 {
-    double y = __builtin_amdgcn_rsq(x);
-    const double h = 0.5 * x;
-    double t = fma(-h * y, y, 0.5);
-    y = fma(y, t, y);
-    t = fma(-h * y, y, 0.5);
-    return fma(y, t, y);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 template <int L>
@@ -153,46 +150,82 @@ __device__ __forceinline__ void boys(double T, const double* __restrict__ table,
     }
 }
 
-// The LDS copy of the coarse rows for order L: lt[k * 12 + j] = F_{L+j}(T_k) / j!.
+// The LDS rows of order L: row k covers T in [k/5, (k+1)/5), T_k = k/5 + 1/10 (a
+// fine row of the table): columns 0..7 the degree-7 polynomial of F_L in
+// x = 10 (T - T_k), |x| <= 1, column 8 exp(-T_k).  The polynomial is the
+// degree-10 Taylor expansion F_L = sum_j F_{L+j}(T_k) (-x/10)^j / j! with its
+// three highest powers replaced by their Chebyshev economisation (error below
+// 0.1^8 / (8! 2^7) F_{L+8} < 2e-15 F_{L+8}(T_k), at most 7e-16 F_L for L <= 4).
+// Ten doubles a row: 16-byte reads of random rows spread over all LDS banks.
 // Every thread of the workgroup calls it; the caller synchronises afterwards.
 template <int L>
 __device__ __forceinline__ void boys_lds_fill(const double* __restrict__ table, double* lt)
 {
-    static_assert(L + VLX_BOYS_CTERMS - 1 < VLX_BOYS_NCOL, "coarse rows hold F_0..F_15");
-    constexpr double inv_fact[VLX_BOYS_CTERMS] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720,
-                                                  1.0 / 5040, 1.0 / 40320, 1.0 / 362880, 1.0 / 3628800,
-                                                  1.0 / 39916800};
-    for (int t = threadIdx.x; t < VLX_BOYS_CROWS * VLX_BOYS_CTERMS; t += blockDim.x) {
-        const int r = t / VLX_BOYS_CTERMS, j = t - r * VLX_BOYS_CTERMS;
-        lt[t] = table[VLX_BOYS_COARSE_OFF + r * VLX_BOYS_NCOL + L + j] * inv_fact[j];
+    static_assert(L + 10 < VLX_BOYS_NCOL - 1, "fine rows hold F_0..F_14");
+    for (int r = threadIdx.x; r < VLX_BOYS_LROWS; r += blockDim.x) {
+        const double* row = table + (10 * r + 5) * VLX_BOYS_NCOL;
+        double c[11], f = 1.0;
+#pragma unroll
+        for (int j = 0; j <= 10; ++j) {
+            c[j] = row[L + j] * f;
+            f *= -0.1 / (double)(j + 1);
+        }
+        c[8] += c[10] * (1280.0 / 512.0);
+        c[6] -= c[10] * (1120.0 / 512.0);
+        c[4] += c[10] * (400.0 / 512.0);
+        c[2] -= c[10] * (50.0 / 512.0);
+        c[0] += c[10] * (1.0 / 512.0);
+        c[7] += c[9] * (576.0 / 256.0);
+        c[5] -= c[9] * (432.0 / 256.0);
+        c[3] += c[9] * (120.0 / 256.0);
+        c[1] -= c[9] * (9.0 / 256.0);
+        c[6] += c[8] * (256.0 / 128.0);
+        c[4] -= c[8] * (160.0 / 128.0);
+        c[2] += c[8] * (32.0 / 128.0);
+        c[0] -= c[8] * (1.0 / 128.0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) lt[r * VLX_BOYS_LCOLS + j] = c[j];
+        lt[r * VLX_BOYS_LCOLS + 8] = row[15];
     }
 }
 
-// F_0..F_L from the LDS copy of the coarse rows (T < VLX_BOYS_TMAX), exp(-T)
-// and downward recursion; the T >= VLX_BOYS_TMAX branch is that of boys<L>.
+// F_0..F_L from the LDS rows (T < VLX_BOYS_TMAX): F_L by its polynomial,
+// exp(-T) = exp(-T_k) exp(-x/10) (degree 8, economised from degree 10: error
+// 1e-17) and downward recursion; the T >= VLX_BOYS_TMAX branch is that of
+// boys<L>.
 template <int L>
 __device__ __forceinline__ void boys_lds(double T, const double* lt, double* F)
 {
     if (T < VLX_BOYS_TMAX) {
-        const int k = (int)(T * VLX_BOYS_INV_CDT + 0.5);
-        const double nd = (double)k * VLX_BOYS_CDT - T;   // -(T - T_k)
-        const double* row = lt + k * VLX_BOYS_CTERMS;
-        double s = row[VLX_BOYS_CTERMS - 1];
+        const int k = (int)(T * 5.0);
+        const double x = fma(T, 10.0, -(double)(2 * k + 1));
+        const double* row = lt + k * VLX_BOYS_LCOLS;
+        double s = row[7];
 #pragma unroll
-        for (int j = VLX_BOYS_CTERMS - 2; j >= 0; --j) s = fma(s, nd, row[j]);
+        for (int j = 6; j >= 0; --j) s = fma(s, x, row[j]);
         F[L] = s;
         if (L > 0) {
-            const double et = exp(-T);
+            constexpr double t9 = -1e-9 / 362880.0, t10 = 1e-10 / 3628800.0;
+            double e = 1e-8 / 40320.0 + t10 * (1280.0 / 512.0);
+            e = fma(e, x, -1e-7 / 5040.0 + t9 * (576.0 / 256.0));
+            e = fma(e, x, 1e-6 / 720.0 - t10 * (1120.0 / 512.0));
+            e = fma(e, x, -1e-5 / 120.0 - t9 * (432.0 / 256.0));
+            e = fma(e, x, 1e-4 / 24.0 + t10 * (400.0 / 512.0));
+            e = fma(e, x, -1e-3 / 6.0 + t9 * (120.0 / 256.0));
+            e = fma(e, x, 1e-2 / 2.0 - t10 * (50.0 / 512.0));
+            e = fma(e, x, -1e-1 - t9 * (9.0 / 256.0));
+            e = fma(e, x, 1.0 + t10 * (1.0 / 512.0));
+            const double et = row[8] * e;
             const double T2 = 2.0 * T;
 #pragma unroll
             for (int m = L - 1; m >= 0; --m) F[m] = fma(T2, F[m + 1], et) * (1.0 / (2.0 * m + 1.0));
         }
     } else {
-        const double inv_T = rcp_nr(T);
-        F[0] = (0.5 * 1.77245385090551602730) * rsq_nr(T);
+        const double y = rsq_nr(T);
+        F[0] = (0.5 * 1.77245385090551602730) * y;
         if (L > 0) {
             const double et = (double)__expf(-(float)T);
-            const double h = 0.5 * inv_T;
+            const double h = 0.5 * (y * y);
 #pragma unroll
             for (int m = 0; m < L; ++m) F[m + 1] = ((2.0 * m + 1.0) * F[m] - et) * h;
         }

@@ -58,8 +58,8 @@ J_LAYOUT_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "j_lay
 # exchange classes that read the density as D[l][j] ("lj", see emit.emit_k),
 # chosen from per-class timings of both orders on lattice64
 DORDER_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "k_dorder.json")
-# light classes that evaluate the Boys function from coarse rows kept in LDS
-# (see emit.lds_boys_setup), chosen from per-class timings on lattice64
+# light classes that evaluate the Boys function from rows kept in LDS (see
+# emit.lds_boys_setup), chosen from per-class timings
 BOYS_LDS_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "boys_lds.json")
 
 
@@ -84,6 +84,18 @@ def load_rys():
             tab = json.load(f)
     return {kind: {cls: dict(zip(("maxx", "tau", "waves"), v)) for cls, v in tab.get(kind, {}).items()}
             for kind in RYS_KINDS}
+
+
+# single-pass exchange classes: wavefronts per SIMD the registers are allotted
+# for, and the classes without an unmasked body (the file's _doc)
+K_LIGHT_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "k_light.json")
+
+
+def load_k_light():
+    """({class: waves per SIMD}, set of classes that always apply the masks)."""
+    with open(K_LIGHT_TABLE) as f:
+        tab = json.load(f)
+    return dict(tab["waves"]), set(tab["masked"])
 
 
 # Coulomb bra classes with many blocks: a tile is full but for the list's last
@@ -188,6 +200,7 @@ def sources(tiles=None, layouts=None):
             out[fn] = rys_inc(cls, 0, r) + inc + emit.emit_j(
                 cls, kt=tiles.get(fn), layout=jlayouts.get(cls, "reg"), lds_boys=cls in blds[fam],
                 wpg=int(wpg[fam].get(cls, 1)), rys=r, pack=ab not in J_UNPACKED, **kw)
+    kwaves, kmasked = load_k_light()
     for cls in k_classes():
         for pre, kw in (("k", {}), ("km", dict(mixed=True)), ("kb", dict(batched=True)),
                         ("kbm", dict(batched=True, mixed=True))):
@@ -196,7 +209,8 @@ def sources(tiles=None, layouts=None):
             r = None if kw.get("mixed") else rys["K"].get(cls)
             out[fn] = rys_inc(cls, 0, r) + inc + emit.emit_k(
                 cls, kt=tiles.get(fn), layout=layouts.get(cls, "reg"), dorder=dorders.get(cls, "jl"),
-                lds_boys=cls in blds[fam], wpg=int(wpg[fam].get(cls, 1)), rys=r, pack=True, **kw)
+                lds_boys=cls in blds[fam], wpg=int(wpg[fam].get(cls, 1)), rys=r, pack=True,
+                waves=kwaves.get(cls, 0), unmask=cls not in kmasked, **kw)
     gp = load_grad_passes()
     for ab, cd in j_classes():
         cls = j_name(ab, cd)

@@ -39,16 +39,16 @@ KET_TILE = 64
 # LDS a single-wavefront workgroup may use without lowering the occupancy of a
 # kernel that needs all 512 registers (160 KB per CU / 4 SIMDs)
 LDS_PER_WAVE_FULL_REGS = 40960
-# ket tile of the kernels that keep the coarse Boys rows in LDS (9.7 KB)
+# ket tile of the kernels that keep Boys rows in LDS (16 KB)
 LDS_BOYS_KT = 16
 
 
 def lds_boys_setup(L):
-    """Kernel-start copy of the coarse Boys rows of order L into LDS (every
+    """Kernel-start construction of the Boys rows of order L in LDS (every
     thread of the workgroup, then a barrier); quartets then evaluate F_L with
     vlxmi::boys_lds instead of gathering a table row per lane."""
-    assert L + 11 <= 15, "coarse rows hold F_0..F_15"
-    return ["    __shared__ double lboys[VLX_BOYS_CROWS * VLX_BOYS_CTERMS];",
+    assert L + 10 <= 14, "fine rows hold F_0..F_14"
+    return ["    __shared__ double lboys[VLX_BOYS_LROWS * VLX_BOYS_LCOLS];",
             "    vlxmi::boys_lds_fill<%d>(boys_func_table, lboys);" % L,
             "    __syncthreads();"]
 # ket record (LDS, doubles): 0 screening bound, 1 eta, 2 1/eta, 3-5 Q, 6-8 QC,
@@ -76,7 +76,7 @@ def quartet_prologue(L, ty_geo="double", omega=False, ind="    ", lds_boys=False
     o.append("const double rho = zeta * eta * inv_S4;")
     o.append("const double PQ_x = Q_x - P_x, PQ_y = Q_y - P_y, PQ_z = Q_z - P_z;")
     o.append("double Tb = rho * (PQ_x * PQ_x + PQ_y * PQ_y + PQ_z * PQ_z);")
-    o.append("double Lambda = (1.12837916709551257390 * rS4) * (sq_zeta * sq_eta);")
+    o.append("double Lambda = rS4 * ((1.12837916709551257390 * sq_zeta) * sq_eta);")
     if omega:
         o.append("double d2 = 1.0;")
         o.append("if (omega != 0.0) { d2 = omega * omega / (rho + omega * omega); Tb *= d2; Lambda *= sqrt(d2); }")
@@ -311,23 +311,19 @@ def _dag_lines(dag):
     return out
 
 
-def pack_decls(ind, rem, lane="lane"):
+def pack_decls(ind, rem, lane="lane", halve=True):
     """How a tile's lanes are shared out in a packed kernel: the largest power
     of two W of bra blocks that is not mostly empty takes the wavefront's
     lanes, which form G = 64 / W groups; group ``slot`` of lanes evaluates
     every G-th ket record.  ``rem`` is the (uniform) number of blocks left.
     W is the power of two that holds ``rem`` (at most 64), halved when the
     blocks would fill at most three quarters of it: the rest then follow in a
-    narrower tile."""
-    return [ind + "uint32_t wsh = %s > 32 ? 6 : (%s > 1 ? 32 - __clz(%s - 1) : 0);" % (rem, rem, rem),
-            ind + "if (wsh > 3 && %s * 4 <= (3u << wsh)) --wsh;" % rem,
-            ind + "const uint32_t slot = %s >> wsh, G = 64u >> wsh, jl = %s & ((1u << wsh) - 1);" % (lane, lane)]
-
-
-def pack_decls1(ind, rem):
-    """As pack_decls for a kernel whose tile is fixed (a Coulomb bra tile of at
-    most 64 blocks): W is the power of two that holds ``rem`` blocks."""
-    return [x for x in pack_decls(ind, rem) if "--wsh" not in x]
+    narrower tile (``halve``; not for a Coulomb bra tile, which is fixed).
+    There are never more groups than staged records (KT)."""
+    return ([ind + "uint32_t wsh = %s > 32 ? 6 : (%s > 1 ? 32 - __clz(%s - 1) : 0);" % (rem, rem, rem)]
+            + ([ind + "if (wsh > 3 && %s * 4 <= (3u << wsh)) --wsh;" % rem] if halve else [])
+            + [ind + "while ((64u >> wsh) > KT) ++wsh;",
+               ind + "const uint32_t slot = %s >> wsh, G = 64u >> wsh, jl = %s & ((1u << wsh) - 1);" % (lane, lane)])
 
 
 def ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=False, pack=False):
@@ -339,9 +335,9 @@ def ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=Fals
     sb + 1, .. sb + G - 1 (the lanes of a group beyond the tile's end wait)."""
     if pack:
         q = [ind + "for (; sb < nt; sb += G) {",
-             ind + "    const uint32_t s = sb + slot < nt ? sb + slot : sb;",
+             ind + "    const uint32_t s = sb + slot;",
              ind + "    const double* R = ket + s * REC;",
-             ind + "    bool live = %s && sb + slot < nt;" % act,
+             ind + "    bool live = %s && s < nt;" % act,
              ind + "    if (live && %s) live = %s = false;" % (screen, act)]
     else:
         q = [ind + "for (; s < nt; ++s) {",
@@ -361,6 +357,37 @@ def ket_loop(ind, act, screen, bound, header, body, ty, check_lo, lo, count=Fals
     q += body(ty, ind + "        ")
     q += [ind + "    }", ind + "}"]
     return q
+
+
+# A single-pass kernel with at most this many component quartets evaluates them
+# all before it digests (a register pair each); one with more digests every
+# component as it appears.
+WHOLE_MAX = 9
+
+
+def whole_body(ind, rec, comps, recursion, digest):
+    """Body of a single-pass quartet with the masks left out when every
+    component of every live lane's quartet passes the screen (one uniform test:
+    a masked term costs four instructions, an unmasked one), else with them.
+    ``recursion(terms)``: the recursion's lines, ``terms(dag, i)`` being called
+    where component i can be formed; ``digest(i, x, masked)``: its digestion."""
+    test = ind + "const bool whole = __all(R[%d] > taumax);" % (rec - 1)
+    if len(comps) <= WHOLE_MAX:
+        names = {}
+
+        def keep(i, x):
+            names[i] = x
+            return []
+        out = recursion(keep) + [test, ind + "if (whole) {"]
+        for masked in (False, True):
+            out += [ind + "    " + l for i in comps for l in digest(i, names[i], masked)]
+            out.append(ind + ("}" if masked else "} else {"))
+        return out
+    out = [test, ind + "if (whole) {"]
+    for masked in (False, True):
+        out += ["    " + l for l in recursion(lambda i, x, m=masked: digest(i, x, m))]
+        out.append(ind + ("}" if masked else "} else {"))
+    return out
 
 
 def rys_ket_loop(ind, screen, header, body, count=False):
@@ -598,16 +625,16 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
             o.append("    for (uint32_t w = blockIdx.x * WPG + wave; w < nwork; w += gridDim.x * WPG) {")
         o.append("    const uint32_t bra_end = work[4 * w + 1] < nbra ? work[4 * w + 1] : nbra;")
         if pack:
-            o += pack_decls1("    ", "(bra_end - work[4 * w])")
+            o += pack_decls("    ", "(bra_end - work[4 * w])", halve=False)
         o.append("    const uint32_t bb = work[4 * w] + %s;" % ("jl" if pack else "lane"))
         o.append("    const uint32_t k_begin = work[4 * w + 2];")
         o.append("    const uint32_t k_end = work[4 * w + 3] < nket ? work[4 * w + 3] : nket;")
         o.append("    const bool own = bb < bra_end;")
     else:
-        tile = "blockIdx.x" if wpg == 1 else "(blockIdx.x * WPG + wave)"
+        tile = "blockIdx.x" if wpg == 1 else "(blockIdx.x * (blockDim.x >> 6) + wave)"
         if pack:
             o.append("    const uint32_t left = nbra > %s * TILE_SIZE_J ? nbra - %s * TILE_SIZE_J : 0;" % (tile, tile))
-            o += pack_decls1("    ", "left")
+            o += pack_decls("    ", "left", halve=False)
         o.append("    const uint32_t bb = %s * TILE_SIZE_J + %s;" % (tile, "jl" if pack else "lane"))
         o.append("    const uint32_t chunk = (nket + gridDim.y - 1) / gridDim.y;")
         o.append("    const uint32_t k_begin = blockIdx.y * chunk;")
@@ -617,8 +644,9 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("    bool active = own;")
     o.append("    double zeta = 1.0, sq_zeta = 1.0, inv_S1 = 1.0, P_x = 0.0, P_y = 0.0, P_z = 0.0;")
     o.append("    double PA_x = 0.0, PA_y = 0.0, PA_z = 0.0, AB_x = 0.0, AB_y = 0.0, AB_z = 0.0;")
-    o.append("    double qmax = 0.0%s;" % (", taumax = 0.0" if rys else ""))
     jsl = plan_slices(la, lb, lc, ld, "J")
+    whole = rys is not None or len(jsl) == 1
+    o.append("    double qmax = 0.0%s;" % (", taumax = 0.0" if whole else ""))
     if rys:
         assert not mixed, "Rys bodies are for the FP64 kernels"
         layout, lds_boys, jpairs = rys["tau"], False, False
@@ -661,11 +689,12 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("            const double q = fabs(%s_mat_Q_local[e0 + t]);" % ab)
     o.append("            qmax = fmax(qmax, q);")
     o.append("            tau[%s] = thr / q;" % ("t * TILE_SIZE_J + lane" if jlds else "t"))
-    if rys:
+    if whole:
         # 0/0 (a zero bound at a zero threshold) passes nothing, like infinity
         o.append("            if (%s_pair_data_local[e0 + t] != 0.0) taumax = fmax(taumax, thr / q >= 0.0 ? thr / q : __builtin_inf());" % ab)
     o.append("        }")
     o.append("    }")
+    o.append("    const double qscr = qmax * (1.0 + 1e-13);")
     if mixed:
         o.append("    bool lo_mode = false;")
         if not batched:
@@ -689,7 +718,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("                R[3] = (ak * C_x + al * D_x) * iet; R[4] = (ak * C_y + al * D_y) * iet; R[5] = (ak * C_z + al * D_z) * iet;")
     o.append("                R[6] = (al * iet) * (D_x - C_x); R[7] = (al * iet) * (D_y - C_y); R[8] = (al * iet) * (D_z - C_z);")
     o.append("                R[9] = C_x - D_x; R[10] = C_y - D_y; R[11] = C_z - D_z;")
-    o.append("                double beta = 0.0%s;" % (", qmin = __builtin_inf()" if rys else ""))
+    o.append("                double beta = 0.0%s;" % (", qmin = __builtin_inf()" if whole else ""))
     o.append("                #pragma unroll")
     o.append("                for (int t = 0; t < NCD; ++t) {")
     o.append("                    const double Dkl = %s_mat_D[f0 + t];" % cd)
@@ -701,11 +730,11 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("                    const double qd = fabs(%s_mat_Q[f0 + t] * Dkl);" % cd)
     o.append("                    R[%d + NCD + t] = qd;" % KREC0)
     o.append("                    beta = fmax(beta, qd);")
-    if rys:
+    if whole:
         # a component whose density weight is zero adds nothing, masked or not
         o.append("                    qmin = fmin(qmin, Dkl != 0.0 ? qd : qmin);")
     o.append("                }")
-    if rys:
+    if whole:
         o.append("                R[%d] = qmin;" % (rec - 1))
     o.append("                R[0] = beta;")
     o.append("            }")
@@ -717,6 +746,22 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         lines = quartet_prologue(L, ty_geo=tyq, ind=ind, lds_boys=lds_boys)
         if jlds:
             lines += [ind + "uint32_t lid = lane;", ind + "asm volatile(\"\" : \"+v\"(lid));"]
+        if whole and len(groups) == 1:
+            comps_ = [(ia * nb + ib, ic * nd + idd) for ic in range(nc) for idd in range(nd)
+                      for ia in range(na) for ib in range(nb)]
+            lines += [ind + "const double Dp%d = R[%d], Qd%d = R[%d];" % (t, KREC0 + t, t, KREC0 + ncd + t) for t in range(ncd)]
+
+            def recursion(use):
+                dag = QuartetDAG(la, lb, lc, ld, ty=tyq, rule_vrr="first", rule_hrr="first", prefix="q")
+                for tab, tcd in comps_:
+                    x = dag.X(tri(la)[tab // nb], tri(lb)[tab % nb], tri(lc)[tcd // nd], tri(ld)[tcd % nd])
+                    dag.lines += use((tab, tcd), x)
+                return [ind + x for x in _dag_lines(dag)]
+
+            def digest(i, x, masked):
+                xv = x if tyq == "double" else "double(%s)" % x
+                return ["acc[%d] += %s * Dp%d;" % (i[0], "((Qd%d > tau[%d]) ? %s : 0.0)" % (i[1], i[0], xv) if masked else xv, i[1])]
+            return lines + whole_body(ind, rec, comps_, recursion, digest)
         for isl, group in enumerate(groups):
             if isl:
                 lines += [ind + x for x in launder(L)]
@@ -771,7 +816,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     # measured faster than one loop per pass
     # the FP32 loop of a mixed kernel may run fewer passes (half-size values)
     jsl32 = plan_slices_f32(la, lb, lc, ld, "J") if mixed else jsl
-    jscreen = "qmax * R[0] * (1.0 + 1e-13) <= thr"
+    jscreen = "qscr * R[0] <= thr"
     if rys:
         o += rys_ket_loop("        ", jscreen, KET_HEADER, jrys, count=batched)
     else:
@@ -893,7 +938,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
 # --------------------------------------------------------------------------
 
 def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", lds_boys=False, wpg=1, kpairs=False,
-           rys=None, pack=False):
+           rys=None, pack=False, waves=0, unmask=True):
     """Source of computeExchangeFock{CLS} (or its _mixed / _batched variants) and
     its launcher.  The batched variant is persistent over a list of (i,k) blocks
     of lists that concatenate many molecules; per block, blk_mol gives the
@@ -913,7 +958,10 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     says where the per-lane thresholds and S_ab are kept ("reg" or "lds"),
     "waves" the wavefronts per SIMD the registers are allotted for.  ``pack``:
     a tile of few partners J shares its lanes out among several ket records
-    (pack_decls; Rys kernels always do)."""
+    (pack_decls; Rys kernels always do).  ``waves``: wavefronts per SIMD the
+    registers are allotted for (0: the compiler's choice).  ``unmask``: single-
+    pass kernels test once per quartet whether any component is screened out
+    (whole_body)."""
     pack = pack or rys is not None
     a, b, c, d = cls
     la, lb, lc, ld = LV[a], LV[b], LV[c], LV[d]
@@ -928,6 +976,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     if rys:
         assert not mixed, "Rys bodies are for the FP64 kernels"
         heavy, layout, lds_boys = False, "reg", False
+        waves = rys["waves"]
         kslices = rys_groups(nab, nc, nd, rys["maxx"])
     if heavy and kpairs:
         # one pass per ket component pair (ic, id): the recursion is recomputed
@@ -943,7 +992,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o = []
     assert not (heavy and wpg > 1), "the heavy layouts keep one wavefront per workgroup"
     o.append("__global__ void __launch_bounds__(%s%s)" % ("TILE_SIZE_K" if wpg == 1 else str(64 * wpg),
-                                                         ", %d" % rys["waves"] if rys and rys.get("waves") else ""))
+                                                         ", %d" % waves if waves else ""))
     o.append("%s(%s)" % (name, ",\n    ".join(sig)))
     o.append("{")
     o.append("    constexpr int NA = %d, NB = %d, NC = %d, ND = %d, NAC = %d, NAB = %d, NCD = %d;" % (na, nb, nc, nd, nac, nab, ncd))
@@ -999,7 +1048,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         o.append("    const double* __restrict__ Dm = mat_D_full_AO + mol_D_off[mol];")
         o.append("    const uint32_t nao = mol_naos[mol], aoff = mol_ao_off[mol];")
     else:
-        o.append("    const uint32_t blk = %s;" % ("blockIdx.x" if wpg == 1 else "blockIdx.x * WPG + wave"))
+        o.append("    const uint32_t blk = %s;" % ("blockIdx.x" if wpg == 1 else "blockIdx.x * (blockDim.x >> 6) + wave"))
         o.append("    if ((blk + 1) * NAC > pair_inds_count_for_K_%s) return;" % ac)
         o.append("    const double maxD = %s_max_D;" % bd)
         o.append("    if (!(maxD > 0.0)) return;")
@@ -1040,7 +1089,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("        bool active = jp < nJ;")
     o.append("        double zeta = 1.0, sq_zeta = 1.0, inv_S1 = 1.0, P_x = 0.0, P_y = 0.0, P_z = 0.0;")
     o.append("        double PA_x = 0.0, PA_y = 0.0, PA_z = 0.0, AB_x = 0.0, AB_y = 0.0, AB_z = 0.0;")
-    o.append("        double qij = 0.0%s;" % (", taumax = 0.0" if rys else ""))
+    o.append("        double qij = 0.0%s;" % ("" if heavy else ", taumax = 0.0"))
     if lds_tau:
         o.append("        double* tau = ltau;")
         o.append("        double* Sab = lSab;")
@@ -1069,7 +1118,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                    const uint32_t pos = displ_i[ca] + jp * NB + cb;")
     o.append("                    const double q = fabs(Q_K_%s[pos]);" % ab)
     o.append("                    qij = fmax(qij, q);")
-    if rys:
+    if not heavy:
         # 0/0 (a zero bound at a zero threshold) passes nothing, like infinity
         o.append("                    if (pair_data_K_%s[pos] != 0.0) taumax = fmax(taumax, thr_eff / q >= 0.0 ? thr_eff / q : __builtin_inf());" % ab)
     if lds_tau:
@@ -1089,6 +1138,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         o.append("                cgJ[cb] = %s_prim_aoinds[(jj / NB) + %s_prim_count * (jj %% NB)] - aoff;" % (b, b))
     o.append("            }")
     o.append("        }")
+    o.append("        const double qscr = qij * maxD * (1.0 + 1e-13);")
     if mixed:
         o.append("        bool lo_mode = false;")
     o.append("        for (uint32_t t0 = 0; t0 < nL; t0 += KT) {")
@@ -1107,7 +1157,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                    R[3] = (ak * C_x + al * D_x) * iet; R[4] = (ak * C_y + al * D_y) * iet; R[5] = (ak * C_z + al * D_z) * iet;")
     o.append("                    R[6] = (al * iet) * (D_x - C_x); R[7] = (al * iet) * (D_y - C_y); R[8] = (al * iet) * (D_z - C_z);")
     o.append("                    R[9] = C_x - D_x; R[10] = C_y - D_y; R[11] = C_z - D_z;")
-    o.append("                    double qk = 0.0%s;" % (", qmin = __builtin_inf()" if rys else ""))
+    o.append("                    double qk = 0.0%s;" % ("" if heavy else ", qmin = __builtin_inf()"))
     o.append("                    #pragma unroll")
     o.append("                    for (int cc = 0; cc < NC; ++cc) {")
     o.append("                        #pragma unroll")
@@ -1115,7 +1165,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                            const uint32_t pos = displ_k[cc] + lp * ND + cdd;")
     o.append("                            const double q = fabs(Q_K_%s[pos]);" % cd)
     o.append("                            qk = fmax(qk, q);")
-    if rys:
+    if not heavy:
         # a component whose factor is zero adds nothing, masked or not
         o.append("                            if (pair_data_K_%s[pos] != 0.0) qmin = fmin(qmin, q);" % cd)
     o.append("                            R[%d + cc * ND + cdd] = pair_data_K_%s[pos];" % (KREC0, cd))
@@ -1123,7 +1173,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                        }")
     o.append("                    }")
     o.append("                    R[0] = qk;")
-    if rys:
+    if not heavy:
         o.append("                    R[%d] = qmin;" % (rec - 1))
     o.append("                    #pragma unroll")
     o.append("                    for (int cdd = 0; cdd < ND; ++cdd) {")
@@ -1177,6 +1227,36 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
                 for idd in sorted({d_ for _, d_ in used}):
                     lines.append(ind + "const double Dj%d_%d = %s;"
                                  % (ibb, idd, dread(("rowJ%d" % ibb) if heavy else ("cgJ[%d]" % ibb), idd)))
+        if not heavy:
+            # acc[a,c] += Sab * X * (Sc * D)
+            comps_ = [(ia * nb + ib, ic * nd + idd) for ic in range(nc) for ia in range(na) for ib in range(nb)
+                      for idd in range(nd)]
+            for tcd in range(ncd):
+                lines.append(ind + "const double Qk%d = R[%d];" % (tcd, KREC0 + ncd + tcd))
+                for ib in range(nb):
+                    lines.append(ind + "const double w%d_%d = R[%d] * Dj%d_%d;" % (ib, tcd, KREC0 + tcd, ib, tcd % nd))
+
+            def recursion(use):
+                dag = QuartetDAG(la, lb, lc, ld, ty=tyq, rule_vrr="first", rule_hrr="first", prefix="q")
+                for tab, tcd in comps_:
+                    x = dag.X(tri(la)[tab // nb], tri(lb)[tab % nb], tri(lc)[tcd // nd], tri(ld)[tcd % nd])
+                    dag.lines += use((tab, tcd), x)
+                return [ind + x for x in _dag_lines(dag)]
+
+            def digest(i, x, masked):
+                # the terms of one (a,b|c are summed before S_ab is applied
+                tab, tcd = i
+                xv = x if tyq == "double" else "double(%s)" % x
+                term = "%s * w%d_%d" % ("((Qk%d > tau[%d]) ? %s : 0.0)" % (tcd, tab, xv) if masked else xv, tab % nb, tcd)
+                ic, idd = divmod(tcd, nd)
+                v = "y%d_%d" % (tab, ic)
+                out = ["%s%s %s %s;" % ("double " if idd == 0 else "", v, "=" if idd == 0 else "+=", term)]
+                if idd == nd - 1:
+                    out.append("acc[%d] += Sab[%d] * %s;" % ((tab // nb) * nc + ic, tab, v))
+                return out
+            if not unmask:
+                return lines + recursion(lambda i, x: digest(i, x, True))
+            return lines + whole_body(ind, rec, comps_, recursion, digest)
         # digestion: acc[a,c] += Sab * sum_{b,d} mask * X * Sc * D  (FP64 accumulation)
         for icc, idd in used:
             tcd = icc * nd + idd
@@ -1248,7 +1328,7 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
             lines += [ind + "    }", ind + "}"]
         return lines
 
-    kscreen = "qij * R[0] * maxD * (1.0 + 1e-13) <= thr"
+    kscreen = "qscr * R[0] <= thr"
     kbound = "qij * R[0] * maxD"
     def pacc_io(group, store):
         out = []

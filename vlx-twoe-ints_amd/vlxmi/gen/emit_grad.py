@@ -33,7 +33,7 @@ pass or in one pass per ket-first-index component, a per-class choice
 from __future__ import annotations
 
 from .emit import (KET_HEADER, KET_TILE, KREC0, LV, NC, _argnames, _dag_lines, _strip_restrict,
-                   j_signature, k_signature, ket_loops, launder, pack_decls, pack_decls1, quartet_prologue, rys_decl, rys_grad_pass,
+                   j_signature, k_signature, ket_loops, launder, pack_decls, quartet_prologue, rys_decl, rys_grad_pass,
                    rys_groups, rys_ket_loop, rys_prologue)
 from .osdag import QuartetDAG, add, tri
 
@@ -136,7 +136,7 @@ def emit_jgrad(cls, passes="one", rys=None):
          "    const uint32_t nbra = %s_prim_pair_count_local / NAB;" % ab,
          "    const uint32_t nket = %s_prim_pair_count / NCD;" % cd,
          "    const uint32_t left = nbra - blockIdx.x * 64;",
-         "\n".join(pack_decls1("    ", "left")),
+         "\n".join(pack_decls("    ", "left", halve=False)),
          "    const uint32_t bb = blockIdx.x * 64 + jl;",
          "    const uint32_t chunk = (nket + gridDim.y - 1) / gridDim.y;",
          "    const uint32_t k_begin = blockIdx.y * chunk;",
@@ -177,6 +177,7 @@ def emit_jgrad(cls, passes="one", rys=None):
     o += ["            wab[%s] = %s_pair_data_local[e0 + t] * %s_mat_D_local[e0 + t] * w;" % (at % "t", ab, ab),
           "        }",
           "    }",
+          "    const double qscr = qmax * (1.0 + 1e-13);",
           "    for (uint32_t t0 = k_begin; t0 < k_end; t0 += KT) {",
           "        if (!__any(active)) break;",
           "        __syncthreads();",
@@ -256,9 +257,9 @@ def emit_jgrad(cls, passes="one", rys=None):
         return lines
 
     if rys:
-        o += rys_ket_loop("        ", "qmax * R[0] * (1.0 + 1e-13) <= thr", KET_HEADER, rys_body)
+        o += rys_ket_loop("        ", "qscr * R[0] <= thr", KET_HEADER, rys_body)
     else:
-        o += ket_loops("        ", "active", "qmax * R[0] * (1.0 + 1e-13) <= thr", "qmax * R[0]", KET_HEADER, body, False, "lo_mode", count=False, pack=True)
+        o += ket_loops("        ", "active", "qscr * R[0] <= thr", "qmax * R[0]", KET_HEADER, body, False, "lo_mode", count=False, pack=True)
     o += ["    }",
           "    for (int g = 0; g < 6; ++g) for (uint32_t off = 1u << wsh; off < 64; off <<= 1) gacc[g] += __shfl_xor(gacc[g], off, 64);",
           "    if (own && slot == 0) {",
@@ -413,6 +414,7 @@ def emit_kgrad(cls, passes="one", rys=None, centres=False):
             o.append("                cgJ[cb] = %s_prim_aoinds[(jj / NB) + %s_prim_count * (jj %% NB)];" % (b, b))
         o += ["            }",
               "        }",
+              "        const double qscr = qij * maxD * (1.0 + 1e-13);",
               "        for (uint32_t t0 = 0; t0 < nL; t0 += KT) {",
               "            if (!__any(active)) break;",
               "            __syncthreads();",
@@ -510,9 +512,9 @@ def emit_kgrad(cls, passes="one", rys=None, centres=False):
             return lines
 
         if rys:
-            o += rys_ket_loop("            ", "qij * R[0] * maxD * (1.0 + 1e-13) <= thr", KET_HEADER, rys_body)
+            o += rys_ket_loop("            ", "qscr * R[0] <= thr", KET_HEADER, rys_body)
         else:
-            o += ket_loops("            ", "active", "qij * R[0] * maxD * (1.0 + 1e-13) <= thr", "qij * R[0] * maxD",
+            o += ket_loops("            ", "active", "qscr * R[0] <= thr", "qij * R[0] * maxD",
                            KET_HEADER, body, False, "lo_mode", count=False, pack=True)
         o += ["        }",
               "    }",
