@@ -210,15 +210,23 @@ class FockEngine:
         e1.record(self.torch.cuda.current_stream(self.dev.device))
         self.timer.append((name, e0, e1))
 
-    def _ket_split(self, nbra_blocks, nket_blocks):
+    def _ket_split(self, nbra_blocks, nket_blocks, ncomp=1):
         """Ket-list chunks per Coulomb launch: enough workgroups (one wavefront
         each) for about ``target_waves`` waves, at least 64 ket blocks per
-        chunk.  The light classes wait on the Boys-table gathers; 32768 waves
+        chunk.  The light classes wait on their LDS and table reads; 32768 waves
         (128 per CU over the launch) hide that latency where 2048 did not
-        (lattice64 J build 1.40 s -> 1.11 s)."""
+        (lattice64 J build 1.40 s -> 1.11 s).  ``ncomp``, the component quartets
+        per ket block: from 9 on, the chunks may be as many times shorter (down
+        to 4 blocks, 2 where even those leave SIMDs idle), since a wavefront's
+        time per ket block grows with them and its set-up does not; from 27 on a
+        quarter of the waves is enough.  J of 12 atoms s/p/d 22.8 ms with chunks
+        of 64, 4.2 so; 36 atoms 99.6 and 89.4."""
         tiles = max(1, (nbra_blocks + 63) // 64)
-        s = max(1, -(-self.target_waves // tiles))
-        return int(min(s, max(1, nket_blocks // 64)))
+        waves = self.target_waves if ncomp < 27 else self.target_waves // 4
+        chunk = max(4, min(64, 64 * 9 // ncomp))
+        if ncomp > 144 and tiles * (nket_blocks // 4) < 1024:
+            chunk = 2                  # fewer wavefronts than SIMDs
+        return int(min(max(1, -(-waves // tiles)), max(1, nket_blocks // chunk)))
 
     def bra_slice(self, ab, blocks):
         """The bra list of pair class ``ab`` restricted to the primitive-pair
@@ -272,7 +280,7 @@ class FockEngine:
                      bra["first"].data_ptr(), bra["second"].data_ptr(), bra["pair_data"].data_ptr(), bra["count"],
                      ket["first"].data_ptr(), ket["second"].data_ptr(), ket["pair_data"].data_ptr(), ket["count"],
                      self.dev.boys_table.data_ptr(), self.dev.boys_ft.data_ptr(), self.thr]
-            split = self._ket_split(bra["nblk"], self.jl[cd]["nblk"])
+            split = self._ket_split(bra["nblk"], self.jl[cd]["nblk"], bra["nab"] * self.jl[cd]["nab"])
             mixed = use_mixed("J", cls, self.precision, self.mixed_policy)
             name = "computeCoulombFock" + cls.upper() + ("_mixed" if mixed else "")
             if mixed:

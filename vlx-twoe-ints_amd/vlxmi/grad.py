@@ -141,7 +141,7 @@ class GradientEngine:
                      bra["first"].data_ptr(), bra["second"].data_ptr(), bra["pair_data"].data_ptr(), bra["count"],
                      ket["first"].data_ptr(), ket["second"].data_ptr(), ket["pair_data"].data_ptr(), ket["count"],
                      self.dev.boys_table.data_ptr(), self.dev.boys_ft.data_ptr(), e.thr]
-            split = e._ket_split(bra["nblk"], e.jl[cd]["nblk"])
+            split = e._ket_split(bra["nblk"], e.jl[cd]["nblk"], bra["nab"] * e.jl[cd]["nab"])
             name = "computeCoulombGradient" + cls.upper()
             ev = e._ev_start()
             check(getattr(L, "vlxmi_launch_" + name)(*args, split, self.dev.stream_ptr()), name)
