@@ -86,6 +86,20 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The sum of v over the workgroup's W wavefronts, lane by lane, in wavefront
+// order (buf: W * 64 doubles of LDS).  Every thread calls it.
+template <int W>
+__device__ __forceinline__ double team_sum(double v, double* buf)
+{
+    __syncthreads();
+    buf[threadIdx.x] = v;
+    __syncthreads();
+    double s = buf[threadIdx.x & 63];
+#pragma unroll
+    for (int k = 1; k < W; ++k) s += buf[k * 64 + (threadIdx.x & 63)];
+    return s;
+}
+
 // 1/x and 1/sqrt(x) for positive, normal x well inside the double range (the
 // Gaussian exponent sums and Boys arguments these are used on): the hardware
 // estimate (relative error below 2^-22) refined by one third-order step, which

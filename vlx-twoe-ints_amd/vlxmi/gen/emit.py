@@ -577,6 +577,11 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     la, lb, lc, ld = LV[a], LV[b], LV[c], LV[d]
     na, nb, nc, nd = NC[a], NC[b], NC[c], NC[d]
     pack = pack or rys is not None
+    # batched kernels of several wavefronts per workgroup work on one item
+    # together: wavefront w takes every wpg-th ket tile of the item's range, so
+    # the longest item (a bra tile of the largest molecule against its whole
+    # ket list) does not outlast the rest of the launch
+    team = batched and wpg > 1
     ab, cd = a + b, c + d
     nab, ncd = na * nb, nc * nd
     L = la + lb + lc + ld
@@ -619,10 +624,9 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("    const uint32_t nket = %s_prim_pair_count / NCD;" % cd)
     if batched:
         o += count_decl()
-        if wpg == 1:
-            o.append("    for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {")
-        else:
-            o.append("    for (uint32_t w = blockIdx.x * WPG + wave; w < nwork; w += gridDim.x * WPG) {")
+        if team:
+            o.append("    __shared__ double team_buf[WPG * 64];")
+        o.append("    for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {")
         o.append("    const uint32_t bra_end = work[4 * w + 1] < nbra ? work[4 * w + 1] : nbra;")
         if pack:
             o += pack_decls("    ", "(bra_end - work[4 * w])", halve=False)
@@ -699,7 +703,10 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         o.append("    bool lo_mode = false;")
         if not batched:
             o += count_decl()
-    o.append("    for (uint32_t t0 = k_begin; t0 < k_end; t0 += KT) {")
+    if team:
+        o.append("    for (uint32_t t0 = k_begin + wave * KT; t0 < k_end; t0 += WPG * KT) {")
+    else:
+        o.append("    for (uint32_t t0 = k_begin; t0 < k_end; t0 += KT) {")
     o.append("        if (!__any(active)) break;")
     o.append("        " + sync(wpg))
     o.append("        {")
@@ -832,7 +839,10 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         o.append("        for (uint32_t off = 1u << wsh; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);")
         o.append("        %s = v;" % ("lacc[t * TILE_SIZE_J + lane]" if jlds else "acc[t]"))
         o.append("    }")
-    o.append("    if (own%s) {" % (" && slot == 0" if pack else ""))
+    if team:
+        o.append("    #pragma unroll")
+        o.append("    for (int t = 0; t < NAB; ++t) acc[t] = vlxmi::team_sum<WPG>(acc[t], team_buf);")
+    o.append("    if (own%s%s) {" % (" && slot == 0" if pack else "", " && wave == 0" if team else ""))
     o.append("        const uint32_t e0 = bb * NAB;")
     o.append("        #pragma unroll")
     o.append("        for (int t = 0; t < NAB; ++t) {")
@@ -878,8 +888,7 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         o += checks
         o.append("    if (nwork == 0) return VLXMI_OK;")
         o.append("    if (!work) return VLXMI_ERR_ARG;")
-        o.append("    const uint32_t max_wg = (nwork + %d) / %d;" % (wpg - 1, wpg))
-        o.append("    if (n_workgroups == 0 || n_workgroups > max_wg) n_workgroups = max_wg;")
+        o.append("    if (n_workgroups == 0 || n_workgroups > nwork) n_workgroups = nwork;")
         o.append("    dim3 grid(n_workgroups);")
         o.append("    hipLaunchKernelGGL(%s, grid, dim3(%d), 0, (hipStream_t)stream, %s);" % (name, 64 * wpg, ", ".join(args)))
         o.append("    return (int)hipGetLastError();")
