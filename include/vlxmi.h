@@ -7,6 +7,7 @@
 #include <stddef.h>
 #include <stdint.h>
 #include "vlxmi_kernels.h"
+#include "vlxmi_prep.h"
 #ifdef __cplusplus
 extern "C" {
 #endif

@@ -29,7 +29,7 @@ import numpy as np
 from . import pairs as P
 from .basis import NCART
 from .policy import use_mixed
-from .runtime import Device, check, lib
+from .runtime import KET_RANK_MAX, Device, KetClass, check, lib
 
 
 class FockEngine:
@@ -99,11 +99,30 @@ class FockEngine:
                                I=d.tensor(ik.I.astype(np.uint32)), K=d.tensor(ik.K.astype(np.uint32)),
                                nblk=int(ik.I.size))
         self._build_assembly()
+        self._ket_setup()
         # AO index sets per angular type (for maxD_bd)
         self.ao_of_type = []
         for p in fl.prims:
             self.ao_of_type.append(d.tensor(np.unique(p.aoinds.ravel()).astype(np.int64)) if p is not None else None)
         self.setup_s = time.time() - t0
+
+    def _ket_setup(self):
+        """The resident Coulomb lists as vlxmi_ket_bounds / vlxmi_ket_order take
+        them, and the angular type of every Cartesian AO."""
+        cls = (KetClass * len(self.jl))()
+        ent = blk = 0
+        for c, (pc, j) in zip(cls, self.jl.items()):
+            for f in ("ao_first", "ao_second", "keep", "mat_Q", "pair_data", "first", "second"):
+                setattr(c, f, j[f].data_ptr())
+            c.nblk, c.entry_offset, c.block_offset, c.nab = j["nblk"], ent, blk, j["nab"]
+            ent += j["count"]
+            blk += j["nblk"]
+        self._ket_cls, self._ket_entries, self._ket_blocks = cls, ent, blk
+        aotype = np.zeros(self.naos, dtype=np.uint8)
+        for p in self.fl.prims:
+            if p is not None:
+                aotype[p.aoinds.ravel()] = p.l
+        self.ao_type = self.dev.tensor(aotype)
 
     # ------------------------------------------------------------------ assembly
     def _build_assembly(self):
@@ -146,6 +165,16 @@ class FockEngine:
     def _cat(self, m, order, counts):
         t = self.torch
         parts = [m[pc] if pc in m else t.zeros(counts[pc], dtype=t.float64, device=self.dev.device) for pc in order]
+        if parts and parts[0]._base is not None:
+            # the slices of one buffer in order (run_J, run_K over all classes)
+            whole, o = parts[0]._base, 0
+            for p in parts:
+                if p._base is not whole or p.data_ptr() != whole.data_ptr() + 8 * o:
+                    break
+                o += p.numel()
+            else:
+                if o == whole.numel() and whole.dim() == 1:
+                    return whole
         return t.cat(parts) if parts else t.zeros(0, dtype=t.float64, device=self.dev.device)
 
     def assemble_J(self, matJ):
@@ -165,33 +194,65 @@ class FockEngine:
         return K.view(n, n)
 
     # ------------------------------------------------------------------ per build
-    def cart_density(self, D_sph):
+    def _density(self, D_sph):
+        """(Cartesian density, max|D| per ordered type pair) of D: the density
+        must fit the bound the lists were screened for and be symmetric to
+        rounding (one host read for the checks and the maxima together); it is
+        made exactly symmetric, as some exchange classes read D_jl as D[l][j]."""
         t = self.torch
         if not t.is_tensor(D_sph):
             D_sph = self.dev.tensor(np.asarray(D_sph, dtype=np.float64))
-        Dc = self.T.t() @ D_sph @ self.T
-        # one device reduction, one host read: the density must fit the bound
-        # the lists were screened for and be symmetric to rounding
-        st = t.stack([Dc.abs().amax(), (D_sph - D_sph.t()).abs().amax(), D_sph.abs().amax()]).cpu().tolist()
-        P.check_density(self.fl, *st)
-        # exactly symmetric: some exchange classes read D_jl as D[l][j]
-        return (0.5 * (Dc + Dc.t())).contiguous()
+        if D_sph.dim() != 2:
+            raise ValueError("density must be a matrix, got %d dimensions" % D_sph.dim())
+        D_sph = D_sph.detach()
+        Dc = (self.T.t() @ D_sph @ self.T).contiguous()
+        Ds = D_sph.contiguous()
+        out, st = t.empty_like(Dc), t.empty(12, dtype=t.float64, device=Dc.device)
+        check(lib().vlxmi_density_stats(Dc.data_ptr(), self.ao_type.data_ptr(), self.naos, Ds.data_ptr(), Ds.shape[0],
+                                        out.data_ptr(), st.data_ptr(), self.dev.stream_ptr()), "density_stats")
+        st = st.cpu().tolist()
+        P.check_density(self.fl, *st[:3])
+        types = [l for l in range(3) if self.fl.prims[l] is not None]
+        return out, {"spd"[b] + "spd"[d]: st[3 + 3 * b + d] for b in types for d in types}
+
+    def cart_density(self, D_sph):
+        return self._density(D_sph)[0]
 
     def prepare_kets(self, Dc):
         """mat_D per J list and the ket-ordered copies (device); ``mat_D_bra``
         keeps mat_D in the resident (bra) order."""
         t = self.torch
+        L, st, n = lib(), self.dev.stream_ptr(), self._ket_entries
+        f64 = t.empty((4, n), dtype=t.float64, device=Dc.device)        # mat_D (bra order), then the ket copies
+        ints = t.empty((2, n), dtype=t.int32, device=Dc.device)
+        beta = t.empty(self._ket_blocks, dtype=t.float64, device=Dc.device)
+        cls = type(self._ket_cls).from_buffer_copy(self._ket_cls)
+        Dc = Dc.contiguous()
+        if n:
+            check(L.vlxmi_ket_bounds(cls, len(cls), Dc.data_ptr(), self.naos, f64[0].data_ptr(), beta.data_ptr(), st), "ket_bounds")
+            orders = []
+            for c in cls:
+                if c.nblk > KET_RANK_MAX:
+                    b = beta[c.block_offset: c.block_offset + c.nblk]
+                    orders.append(t.sort(b, descending=True, stable=True).indices)
+                    c.order = orders[-1].data_ptr()
+            check(L.vlxmi_ket_order(cls, len(cls), beta.data_ptr(), f64[0].data_ptr(), ints[0].data_ptr(), ints[1].data_ptr(),
+                                    f64[1].data_ptr(), f64[2].data_ptr(), f64[3].data_ptr(), st), "ket_order")
         kets = {}
-        for pc, j in self.jl.items():
-            mD = Dc[j["ao_first"], j["ao_second"]] * j["keep"].to(t.float64)
-            nab = j["nab"]
-            beta = (j["mat_Q"] * mD).abs().view(-1, nab).amax(dim=1)
-            order = t.sort(beta, descending=True, stable=True).indices
-            ent = (order[:, None] * nab + t.arange(nab, device=Dc.device)[None, :]).reshape(-1)
-            kets[pc] = dict(first=j["first"][ent].contiguous(), second=j["second"][ent].contiguous(),
-                            pair_data=j["pair_data"][ent].contiguous(), mat_Q=j["mat_Q"][ent].contiguous(),
-                            mat_D=mD[ent].contiguous(), count=j["count"], mat_D_bra=mD)
+        for c, (pc, j) in zip(cls, self.jl.items()):
+            a, b = c.entry_offset, c.entry_offset + j["count"]
+            kets[pc] = dict(first=ints[0, a:b], second=ints[1, a:b], pair_data=f64[1, a:b], mat_Q=f64[2, a:b],
+                            mat_D=f64[3, a:b], count=j["count"], mat_D_bra=f64[0, a:b])
         return kets
+
+    def _outputs(self, order, counts, dv):
+        """Zeroed outputs of every class, slices of one buffer."""
+        buf = self.torch.zeros(sum(counts[pc] for pc in order), dtype=self.torch.float64, device=dv)
+        out, o = {}, 0
+        for pc in order:
+            out[pc] = buf[o: o + counts[pc]]
+            o += counts[pc]
+        return out
 
     def _ev_start(self):
         if self.timer is None:
@@ -260,7 +321,8 @@ class FockEngine:
         t = self.torch
         L = lib()
         kets = kets or self.prepare_kets(Dc)
-        out = {}
+        whole = classes is None and bra_blocks is None
+        out = self._outputs(self.j_order, {pc: self.jl[pc]["count"] for pc in self.j_order}, Dc.device) if whole else {}
         slices = {}
         for ab, cd in (classes or P.j_classes()):
             if ab not in self.jl or cd not in self.jl:
@@ -308,7 +370,8 @@ class FockEngine:
         t = self.torch
         L = lib()
         maxD = maxD or self.max_D(Dc)
-        out = {}
+        whole = classes is None and ik_blocks is None
+        out = self._outputs(self.k_order, {pc: self.ik[pc]["count"] for pc in self.k_order}, Dc.device) if whole else {}
         slices = {}
         for cls in (classes or P.k_classes()):
             a, b, c, d = cls
@@ -356,22 +419,29 @@ class FockEngine:
                                            self.thr / maxD, out.data_ptr(), self.dev.stream_ptr()), "count_k_quartets")
         return int(out.item())
 
-    def run_JK(self, Dc):
+    def side_stream(self):
+        """The second stream of builds on the current one, or None where they
+        stay on one stream."""
+        t = self.torch
+        if not (self.concurrent and self.timer is None and self.progress is None):
+            return None
+        key = t.cuda.current_stream(self.dev.device).cuda_stream
+        if key not in self._kstreams:
+            self._kstreams[key] = t.cuda.Stream(device=self.dev.device)
+        return self._kstreams[key]
+
+    def run_JK(self, Dc, maxD=None):
         """run_J and run_K; with ``concurrent`` (and no per-launch timer or
         progress callback) the exchange launches run on a second stream that
         forks from and joins the current one."""
         t = self.torch
-        if not (self.concurrent and self.timer is None and self.progress is None):
-            return self.run_J(Dc), self.run_K(Dc)
+        side = self.side_stream()
+        if side is None:
+            return self.run_J(Dc), self.run_K(Dc, maxD=maxD)
         cur = t.cuda.current_stream(self.dev.device)
-        key = cur.cuda_stream
-        if key not in self._kstreams:
-            self._kstreams[key] = t.cuda.Stream(device=self.dev.device)
-        side = self._kstreams[key]
         side.wait_stream(cur)
         mJ = self.run_J(Dc)
         with t.cuda.stream(side):
-            maxD = self.max_D(Dc)
             mK = self.run_K(Dc, maxD=maxD)
         cur.wait_stream(side)
         for v in mK.values():
@@ -394,8 +464,8 @@ class FockEngine:
             self.fasm = FockAssembler(self.dev, jv, jo, nj, kv, ko, n * n)
         if self.precision == "mixed":
             self.reset_counts()
-        Dc = self.cart_density(D_sph)
-        mJ, mK = self.run_JK(Dc)
+        Dc, maxD = self._density(D_sph)
+        mJ, mK = self.run_JK(Dc, maxD)
         vals = t.cat([self._cat(mJ, self.j_order, {pc: self.jl[pc]["count"] for pc in self.j_order}),
                       self._cat(mK, self.k_order, {pc: self.ik[pc]["count"] for pc in self.k_order})])
         G = t.zeros(n * n, dtype=t.float64, device=self.dev.device)
@@ -431,10 +501,10 @@ class FockEngine:
         """J and K in the output basis for density D (device tensors)."""
         if self.precision == "mixed":
             self.reset_counts()
-        Dc = self.cart_density(D_sph)
+        Dc, maxD = self._density(D_sph)
         if not want_k:
             return self.T @ self.assemble_J(self.run_J(Dc)) @ self.T.t(), None
-        mJ, mK = self.run_JK(Dc)
+        mJ, mK = self.run_JK(Dc, maxD)
         J = self.T @ self.assemble_J(mJ) @ self.T.t()
         K = self.T @ self.assemble_K(mK) @ self.T.t()
         return J, K

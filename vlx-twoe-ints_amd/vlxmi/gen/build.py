@@ -586,13 +586,14 @@ def _build(jobs=None, force=False, only=None, verbose=True):
         f.write(device_header_text())
     todo = []
     objs = []
-    hand = ["vlxmi_capi.cpp", "vlxmi_noalloc.cpp", "vlxmi_lists.cpp", "vlxmi_pairs.cpp"]
+    hand = ["vlxmi_capi.cpp", "vlxmi_noalloc.cpp", "vlxmi_lists.cpp", "vlxmi_pairs.cpp", "vlxmi_prep.cpp"]
     flag_key = " ".join(FLAGS)
     dev_hdr = open(os.path.join(CSRC, "vlxmi_device.hpp")).read() + open(os.path.join(CSRC, "vlxmi_status.h")).read()
+    prep_hdr = open(os.path.join(ROOT, "include", "vlxmi_prep.h")).read()
     for fn in hand:
         p = os.path.join(CSRC, fn)
         text = open(p).read()
-        h = hashlib.sha1((text + dev_hdr + flag_key).encode()).hexdigest()[:16]
+        h = hashlib.sha1((text + dev_hdr + prep_hdr + flag_key).encode()).hexdigest()[:16]
         o = os.path.join(OBJ, "%s.%s.o" % (fn, h))
         objs.append(o)
         if force or not os.path.exists(o):

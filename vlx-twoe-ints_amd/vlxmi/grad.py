@@ -206,8 +206,19 @@ class GradientEngine:
         return g.view(self.natoms, 3)
 
     def gradient(self, D_sph, want_k=True):
-        """(gJ, gK) per atom (device tensors, (natoms, 3)) for density D."""
-        Dc = self.eng.cart_density(D_sph)
+        """(gJ, gK) per atom (device tensors, (natoms, 3)) for density D; the
+        exchange part runs on a second stream where the Fock builds' does."""
+        e, t = self.eng, self.torch
+        Dc, maxD = e._density(D_sph)
+        side = e.side_stream() if want_k else None
+        if side is None:
+            gJ = self.assemble(self.run_J(Dc), "J")
+            return gJ, self.assemble(self.run_K(Dc, maxD=maxD), "K") if want_k else None
+        cur = t.cuda.current_stream(self.dev.device)
+        side.wait_stream(cur)
         gJ = self.assemble(self.run_J(Dc), "J")
-        gK = self.assemble(self.run_K(Dc), "K") if want_k else None
+        with t.cuda.stream(side):
+            gK = self.assemble(self.run_K(Dc, maxD=maxD), "K")
+        cur.wait_stream(side)
+        gK.record_stream(cur)              # allocated on the side stream, read on this one
         return gJ, gK

@@ -19,6 +19,14 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "lib
 
 _lib = None
 
+KET_RANK_MAX = 4096          # VLXMI_KET_RANK_MAX (include/vlxmi_prep.h)
+
+
+class KetClass(C.Structure):
+    """vlxmi_ket_class (include/vlxmi_prep.h)."""
+    _fields_ = [(n, C.c_void_p) for n in ("ao_first", "ao_second", "keep", "mat_Q", "pair_data", "first", "second", "order")] \
+        + [(n, C.c_uint64) for n in ("nblk", "entry_offset", "block_offset")] + [("nab", C.c_uint32), ("unused", C.c_uint32)]
+
 
 class VlxmiError(RuntimeError):
     pass
@@ -124,6 +132,9 @@ def lib():
     L.vlxmi_pair_candidates.argtypes = [C.c_uint32, C.c_uint32, P_, C.c_uint32, P_, C.c_uint32] + [P_] * 5 + [P_]
     L.vlxmi_block_absmax.argtypes = [P_, C.c_uint64, C.c_uint32, P_, P_]
     L.vlxmi_kcsr_fill.argtypes = [C.c_uint32, C.c_uint32] + [P_] * 7 + [C.c_uint64] + [P_] * 6
+    L.vlxmi_density_stats.argtypes = [P_, P_, C.c_uint32, P_, C.c_uint32, P_, P_, P_]
+    L.vlxmi_ket_bounds.argtypes = [P_, C.c_uint32, P_, C.c_uint32, P_, P_, P_]
+    L.vlxmi_ket_order.argtypes = [P_, C.c_uint32] + [P_] * 8
     L.vlxmi_noalloc_scratch_doubles.restype = C.c_uint64
     L.vlxmi_noalloc_scratch_doubles.argtypes = []
     L.vlxmi_count_k_quartets.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32] + [C.c_void_p] * 6 + [C.c_double, C.c_void_p, C.c_void_p]
@@ -145,7 +156,8 @@ def exported_symbols():
              "vlxmi_coulomb_fock_noalloc", "vlxmi_noalloc_scratch_doubles", "vlxmi_j_list_to_blocks",
              "vlxmi_ik_list_to_blocks", "vlxmi_k_csr_to_blocks", "vlxmi_scatter_add", "vlxmi_validate_j_list",
              "vlxmi_validate_ik_list", "vlxmi_validate_k_csr", "vlxmi_set_list_validation", "vlxmi_list_validation",
-             "vlxmi_pair_candidates", "vlxmi_block_absmax", "vlxmi_kcsr_fill", "vlxmi_fock_assemble"]
+             "vlxmi_pair_candidates", "vlxmi_block_absmax", "vlxmi_kcsr_fill", "vlxmi_fock_assemble",
+             "vlxmi_density_stats", "vlxmi_ket_bounds", "vlxmi_ket_order"]
     names += ["vlxmi_launch_computeCoulombFock" + (ab + cd).upper() for ab, cd in j_classes()]
     names += ["vlxmi_launch_computeExchangeFock" + c.upper() for c in k_classes()]
     names += ["vlxmi_launch_computeCoulombFock" + (ab + cd).upper() + "_mixed" for ab, cd in j_classes()]
