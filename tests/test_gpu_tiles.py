@@ -98,3 +98,31 @@ def test_gradient_tiles_against_oracle(dev, n):
         for k in ref:
             if ref[k].size:
                 assert np.abs(got[k].cpu().numpy() - ref[k]).max() <= 1e-11 * scale, k
+
+
+def test_exchange_split_under_capture(dev):
+    """An exchange launch over few blocks splits its partners among wavefronts
+    (partial sums in the library's workspace); while a stream is captured it
+    stays unsplit, and the graph gives the same sums on every replay."""
+    from vlxmi.fock import FockEngine
+    print("case: exchange launches in a graph", flush=True)
+    t = dev.torch
+    mol, D = _chain(12)
+    eng = FockEngine(mol, dev=dev)
+    Dc = eng.cart_density(D)
+    maxD = eng.max_D(Dc)
+    for cls in ("ssss", "dpds", "pddd"):
+        ref = eng.run_K(Dc, classes=[cls], maxD=maxD)[cls[0] + cls[2]].clone()
+        s = t.cuda.Stream(device=dev.device)
+        s.wait_stream(t.cuda.current_stream(dev.device))
+        g = t.cuda.CUDAGraph()
+        with t.cuda.stream(s):
+            eng.run_K(Dc, classes=[cls], maxD=maxD)
+        t.cuda.synchronize()
+        with t.cuda.graph(g):
+            out = eng.run_K(Dc, classes=[cls], maxD=maxD)[cls[0] + cls[2]]
+        for _ in range(3):
+            g.replay()
+            t.cuda.synchronize()
+            assert (out - ref).abs().max() <= 1e-12 * max(1.0, float(ref.abs().max()))
+            eng.run_K(Dc, classes=[cls], maxD=maxD)

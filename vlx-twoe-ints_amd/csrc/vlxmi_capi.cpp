@@ -303,6 +303,22 @@ extern "C" int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out)
     return VLXMI_OK;
 }
 
+// As vlxmi_ket_workspace for launches that can do without: an error, with
+// nothing changed and no HIP error left behind, when the stream is being
+// captured or the memory is not to be had.
+extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out)
+{
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        return VLXMI_ERR_ARG;
+    }
+    if (capturing != hipStreamCaptureStatusNone) return VLXMI_ERR_ARG;
+    const int rc = vlxmi_ket_workspace(ndoubles, stream, out);
+    if (rc > 0) (void)hipGetLastError();
+    return rc;
+}
+
 // Frees every ket-split workspace (after a device synchronization).
 extern "C" int vlxmi_release_workspaces(void)
 {

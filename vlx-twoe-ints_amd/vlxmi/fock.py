@@ -271,16 +271,16 @@ class FockEngine:
         e1.record(self.torch.cuda.current_stream(self.dev.device))
         self.timer.append((name, e0, e1))
 
-    def _ket_split(self, nbra_blocks, nket_blocks, ncomp=1):
+    def _ket_split(self, nbra_blocks, nket_blocks, ncomp=1296):
         """Ket-list chunks per Coulomb launch: enough workgroups (one wavefront
         each) for about ``target_waves`` waves, at least 64 ket blocks per
         chunk.  The light classes wait on their LDS and table reads; 32768 waves
         (128 per CU over the launch) hide that latency where 2048 did not
         (lattice64 J build 1.40 s -> 1.11 s).  ``ncomp``, the component quartets
-        per ket block: from 9 on, the chunks may be as many times shorter (down
-        to 4 blocks, 2 where even those leave SIMDs idle), since a wavefront's
-        time per ket block grows with them and its set-up does not; from 27 on a
-        quarter of the waves is enough.  J of 12 atoms s/p/d 22.8 ms with chunks
+        per ket block (by default the heaviest class's): from 9 on, the chunks
+        may be as many times shorter (down to 4 blocks, 2 where even those leave
+        SIMDs idle), since a wavefront's time per ket block grows with them and
+        its set-up does not; from 27 on a quarter of the waves is enough.  J of 12 atoms s/p/d 22.8 ms with chunks
         of 64, 4.2 so; 36 atoms 99.6 and 89.4."""
         tiles = max(1, (nbra_blocks + 63) // 64)
         waves = self.target_waves if ncomp < 27 else self.target_waves // 4

@@ -946,6 +946,26 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
 # K kernel
 # --------------------------------------------------------------------------
 
+def k_split_launch(name, ncomp, ket_count, out_count, max_d, grid, threads, args, out, kt):
+    """Launcher lines of an exchange kernel's ket split.  A short (i,k) list
+    leaves most of the 1024 SIMDs idle while each block's wavefront walks its
+    partners alone: chunks of the ket tiles then run as blocks of their own, as
+    many as give two wavefronts a SIMD (half a wavefront for the classes below
+    27 component quartets, whose blocks are short), at most 16.  Without memory
+    for the partial sums, and while the stream is being captured (growing that
+    memory is not a graph operation), the launch stays unsplit."""
+    return ["    if (!(%s > 0.0)) return VLXMI_OK;" % max_d,
+            "    const uint32_t tiles = (%s + %d) / %d, want = (%du + nblk - 1) / nblk;" % (ket_count, kt - 1, kt, 2048 if ncomp >= 27 else 512),
+            "    const uint32_t split = want < tiles ? (want < 16 ? want : 16) : (tiles < 16 ? tiles : 16);",
+            "    double* part = nullptr;",
+            "    if (split > 1 && vlxmi_try_workspace((size_t)split * %s, stream, &part) == VLXMI_OK) {" % out_count,
+            "        hipLaunchKernelGGL(%s_ks, %s, dim3(%d), 0, (hipStream_t)stream, %s, part);" % (name, grid, threads, args),
+            "        const int rc = (int)hipGetLastError();",
+            "        if (rc != 0) return rc;",
+            "        return vlxmi_ket_split_reduce(part, split, %s, %s, stream);" % (out_count, out),
+            "    }"]
+
+
 def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", lds_boys=False, wpg=1, kpairs=False,
            rys=None, pack=False, waves=0, unmask=True):
     """Source of computeExchangeFock{CLS} (or its _mixed / _batched variants) and
@@ -1000,9 +1020,18 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     ty = "double"
     o = []
     assert not (heavy and wpg > 1), "the heavy layouts keep one wavefront per workgroup"
-    o.append("__global__ void __launch_bounds__(%s%s)" % ("TILE_SIZE_K" if wpg == 1 else str(64 * wpg),
-                                                         ", %d" % waves if waves else ""))
-    o.append("%s(%s)" % (name, ",\n    ".join(sig)))
+    # The plain kernels share one body: chunk y of a ket split (grid.y) takes
+    # every gridDim.y-th ket tile of a block and, with k_partial, stores its
+    # sums at k_partial[y * count + e] for the launcher's ordered reduction.
+    split = not (mixed or batched or heavy)
+    bounds = "__launch_bounds__(%s%s)" % ("TILE_SIZE_K" if wpg == 1 else str(64 * wpg), ", %d" % waves if waves else "")
+    KP = ["double* __restrict__ k_partial"]
+    if split:
+        o.append("static __device__ __forceinline__ void")
+        o.append("%s_body(%s)" % (name, ",\n    ".join(sig + KP)))
+    else:
+        o.append("__global__ void %s" % bounds)
+        o.append("%s(%s)" % (name, ",\n    ".join(sig)))
     o.append("{")
     o.append("    constexpr int NA = %d, NB = %d, NC = %d, ND = %d, NAC = %d, NAB = %d, NCD = %d;" % (na, nb, nc, nd, nac, nab, ncd))
     o.append("    constexpr int KT = %d, REC = %d;" % (LDS_BOYS_KT if lds_boys else (kt or (32 if heavy else KET_TILE)), rec))
@@ -1150,7 +1179,10 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("        const double qscr = qij * maxD * (1.0 + 1e-13);")
     if mixed:
         o.append("        bool lo_mode = false;")
-    o.append("        for (uint32_t t0 = 0; t0 < nL; t0 += KT) {")
+    if split:
+        o.append("        for (uint32_t t0 = blockIdx.y * KT; t0 < nL; t0 += gridDim.y * KT) {")
+    else:
+        o.append("        for (uint32_t t0 = 0; t0 < nL; t0 += KT) {")
     o.append("            if (!__any(active)) break;")
     o.append("            " + sync(wpg))
     o.append("            {")
@@ -1426,7 +1458,13 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("        double v = %s;" % ("lacc[t * TILE_SIZE_K + lane]" if lacc else "acc[t]"))
     o.append("        #pragma unroll")
     o.append("        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);")
-    o.append("        if (lane == 0) mat_K[e0 + t] += v;")
+    if split:
+        o.append("        if (lane == 0) {")
+        o.append("            if (k_partial != nullptr) k_partial[(size_t)blockIdx.y * pair_inds_count_for_K_%s + e0 + t] = v;" % ac)
+        o.append("            else mat_K[e0 + t] += v;")
+        o.append("        }")
+    else:
+        o.append("        if (lane == 0) mat_K[e0 + t] += v;")
     o.append("    }")
     if batched:
         o.append("    " + sync(wpg))
@@ -1435,6 +1473,14 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         o += count_flush()
     o.append("}")
     o.append("")
+    if split:
+        for suffix, params, last in (("", sig, "nullptr"), ("_ks", sig + KP, "k_partial")):
+            o.append("__global__ void %s" % bounds)
+            o.append("%s%s(%s)" % (name, suffix, ",\n    ".join(params)))
+            o.append("{")
+            o.append("    %s_body(%s, %s);" % (name, ", ".join(_argnames(sig)), last))
+            o.append("}")
+            o.append("")
     lsig = _strip_restrict(sig)
     args = _argnames(sig)
     if batched:
@@ -1465,6 +1511,10 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
         o.append("    if (n_workgroups == 0 || n_workgroups > max_wg) n_workgroups = max_wg;")
         o.append("    hipLaunchKernelGGL(%s, dim3(n_workgroups), dim3(%d), 0, (hipStream_t)stream, %s);" % (name, 64 * wpg, ", ".join(args)))
     else:
+        if split:
+            o += k_split_launch(name, nab * ncd, "%s_prim_count" % d, "pair_inds_count_for_K_%s" % ac, "%s_max_D" % bd,
+                                "dim3((nblk + %d) / %d, split)" % (wpg - 1, wpg), 64 * wpg, ", ".join(args), "mat_K",
+                                LDS_BOYS_KT if lds_boys else (kt or KET_TILE))
         o.append("    hipLaunchKernelGGL(%s, dim3((nblk + %d) / %d), dim3(%d), 0, (hipStream_t)stream, %s);" % (name, wpg - 1, wpg, 64 * wpg, ", ".join(args)))
     o.append("    return (int)hipGetLastError();")
     o.append("}")

@@ -33,7 +33,7 @@ pass or in one pass per ket-first-index component, a per-class choice
 from __future__ import annotations
 
 from .emit import (KET_HEADER, KET_TILE, KREC0, LV, NC, _argnames, _dag_lines, _strip_restrict,
-                   j_signature, k_signature, ket_loops, launder, pack_decls, quartet_prologue, rys_decl, rys_grad_pass,
+                   j_signature, k_signature, k_split_launch, ket_loops, launder, pack_decls, quartet_prologue, rys_decl, rys_grad_pass,
                    rys_groups, rys_ket_loop, rys_prologue)
 from .osdag import QuartetDAG, add, tri
 
@@ -324,10 +324,15 @@ def emit_kgrad(cls, passes="one", rys=None, centres=False):
     lds = rys is not None and rys["tau"] == "lds"
     at = "%s * 64 + lane" if lds else "%s"
 
+    bounds = "__launch_bounds__(64%s)" % (", %d" % rys["waves"] if rys and rys.get("waves") else "")
+    KP = ["double* __restrict__ k_partial"]
+
     def kernel(kname, cents):
-        o = ["__global__ void __launch_bounds__(64%s)" % (", %d" % rys["waves"] if rys and rys.get("waves") else ""),
-             "%s(%s)" % (kname, ",\n    ".join(sig)),
-             "{",
+        # the class's own kernel has a ket-split form, as the Fock kernels
+        own = kname == name
+        o = (["static __device__ __forceinline__ void", "%s_body(%s)" % (kname, ",\n    ".join(sig + KP))] if own else
+             ["__global__ void %s" % bounds, "%s(%s)" % (kname, ",\n    ".join(sig))])
+        o += ["{",
              "    constexpr int NA = %d, NB = %d, NC = %d, ND = %d, NAC = %d, NAB = %d, NCD = %d;" % (na, nb, nc, nd, nac, nab, ncd),
              "    constexpr int KT = %d, REC = %d;" % (kt, rec),
              "    __shared__ double ket[KT * REC];",
@@ -415,7 +420,7 @@ def emit_kgrad(cls, passes="one", rys=None, centres=False):
         o += ["            }",
               "        }",
               "        const double qscr = qij * maxD * (1.0 + 1e-13);",
-              "        for (uint32_t t0 = 0; t0 < nL; t0 += KT) {",
+              "        for (uint32_t t0 = %s; t0 < nL; t0 += %sKT) {" % (("blockIdx.y * KT", "gridDim.y * ") if own else ("0", "")),
               "            if (!__any(active)) break;",
               "            __syncthreads();",
               "            {",
@@ -523,10 +528,20 @@ def emit_kgrad(cls, passes="one", rys=None, centres=False):
               "        double v = gacc[g];",
               "        #pragma unroll",
               "        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);",
-              "        if (lane == 0) grad_%s[(size_t)blk * 6 + %d + g] += v;" % (ac, cents[0][2]),
-              "    }",
+              "        if (lane == 0) {" if own else
+              "        if (lane == 0) grad_%s[(size_t)blk * 6 + %d + g] += v;" % (ac, cents[0][2])]
+        if own:
+            o += ["            if (k_partial != nullptr)",
+                  "                k_partial[((size_t)blockIdx.y * (pair_inds_count_for_K_%s / NAC) + blk) * 6 + g] = v;" % ac,
+                  "            else grad_%s[(size_t)blk * 6 + g] += v;" % ac,
+                  "        }"]
+        o += ["    }",
               "}",
               ""]
+        if own:
+            for suffix, params, last in (("", sig, "nullptr"), ("_ks", sig + KP, "k_partial")):
+                o += ["__global__ void %s" % bounds, "%s%s(%s)" % (kname, suffix, ",\n    ".join(params)), "{",
+                      "    %s_body(%s, %s);" % (kname, ", ".join(_argnames(sig)), last), "}", ""]
         return o
 
     # (position, 2 x exponent, first output column) of the centres a kernel covers
@@ -553,6 +568,8 @@ def emit_kgrad(cls, passes="one", rys=None, centres=False):
                  % (lc, ld, c, cd, cd, cd, cd))
     o += ["        if (rc != 0) return rc;",
           "    }"]
+    o += k_split_launch(name, 4 * nab * ncd, "%s_prim_count" % d, "(nblk * 6)", "%s_max_D" % bd, "dim3(nblk, split)", 64,
+                        ", ".join(args), "grad_%s" % ac, kt)
     o += ["    hipLaunchKernelGGL(%s, dim3(nblk), dim3(64), 0, (hipStream_t)stream, %s);" % (name, ", ".join(args)),
           "    return (int)hipGetLastError();",
           "}"]
