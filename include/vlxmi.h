@@ -26,7 +26,7 @@ int vlxmi_boys_table_fill(double* table, double* ft);
 /* out[t*(L+1)+m] = F_m(T[t]), the device Boys function (test probe). */
 int vlxmi_boys_eval(const double* T, uint32_t n, uint32_t L, const double* table, double* out, void* stream);
 
-/* As vlxmi_boys_eval through the table's coarse rows copied to LDS, the
+/* As vlxmi_boys_eval through polynomial rows in LDS made from the table's fine rows, the
  * evaluation some light-class kernels use (L = 0..4; test probe). */
 int vlxmi_boys_eval_coarse(const double* T, uint32_t n, uint32_t L, const double* table, double* out,
                            void* stream);

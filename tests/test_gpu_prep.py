@@ -55,6 +55,29 @@ def test_ket_order_equals_stable_sort(dev, nblk, nab):
                                      f64[1].data_ptr(), f64[2].data_ptr(), f64[3].data_ptr(), st) == -3
 
 
+def test_nan_bound_leads(dev):
+    """A block with a NaN entry keeps NaN as its bound and leads its list, as in
+    a device sort."""
+    from vlxmi.runtime import KetClass, check, lib
+    t = dev.torch
+    D = dev.tensor(np.array([[1.0, np.nan], [2.0, 3.0]]))
+    ao = dev.tensor(np.array([0, 0, 0, 1]))
+    cls = (KetClass * 1)()
+    keep, Q = t.ones(4, dtype=t.bool, device=dev.device), t.ones(4, dtype=t.float64, device=dev.device)
+    second, idx = dev.tensor(np.array([0, 0, 1, 1])), dev.tensor(np.arange(4, dtype=np.uint32))
+    for k, v in dict(ao_first=ao, ao_second=second, keep=keep, mat_Q=Q, pair_data=Q, first=idx, second=idx).items():
+        setattr(cls[0], k, v.data_ptr())
+    cls[0].nblk, cls[0].nab = 2, 2
+    f64, b = t.empty((4, 4), dtype=t.float64, device=dev.device), t.empty(2, dtype=t.float64, device=dev.device)
+    ints = t.empty((2, 4), dtype=t.int32, device=dev.device)
+    st = dev.stream_ptr()
+    check(lib().vlxmi_ket_bounds(cls, 1, D.data_ptr(), 2, f64[0].data_ptr(), b.data_ptr(), st))
+    check(lib().vlxmi_ket_order(cls, 1, b.data_ptr(), f64[0].data_ptr(), ints[0].data_ptr(), ints[1].data_ptr(),
+                                f64[1].data_ptr(), f64[2].data_ptr(), f64[3].data_ptr(), st))
+    assert b[0].item() == 1.0 and t.isnan(b[1]).item()
+    assert ints[0].tolist() == [2, 3, 0, 1]
+
+
 def test_density_maxima_and_checks(dev):
     """The maxima equal FockEngine.max_D of the symmetrised density, which is
     exactly symmetric; densities that were refused still are."""

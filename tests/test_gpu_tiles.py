@@ -126,3 +126,43 @@ def test_exchange_split_under_capture(dev):
             t.cuda.synchronize()
             assert (out - ref).abs().max() <= 1e-12 * max(1.0, float(ref.abs().max()))
             eng.run_K(Dc, classes=[cls], maxD=maxD)
+
+
+def test_exchange_split_two_threads_one_stream(dev):
+    """Two threads launch split exchange classes of different sizes on one
+    stream: each gets the sums it gets alone, bit for bit (a launch and its
+    reduction hold the stream's workspace together)."""
+    import threading
+    from vlxmi.fock import FockEngine
+    print("case: two threads, one stream", flush=True)
+    t = dev.torch
+    work = []
+    for n in (9, 17):
+        mol, D = _chain(n)
+        eng = FockEngine(mol, dev=dev)
+        Dc = eng.cart_density(D)
+        work.append((eng, Dc, eng.max_D(Dc)))
+    classes = ("ssss", "dpds", "pddd", "sdpd")
+
+    def run(w):
+        eng, Dc, maxD = w
+        return [eng.run_K(Dc, classes=[c], maxD=maxD)[c[0] + c[2]].clone() for c in classes]
+
+    alone = [run(w) for w in work]
+    t.cuda.synchronize()
+    got = [[], []]
+
+    def loop(i):
+        for _ in range(6):
+            got[i].append(run(work[i]))
+
+    ts = [threading.Thread(target=loop, args=(i,)) for i in range(2)]
+    for x in ts:
+        x.start()
+    for x in ts:
+        x.join(60)
+    assert not any(x.is_alive() for x in ts)
+    t.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 6
+        assert all(t.equal(a, b) for r in got[i] for a, b in zip(r, alone[i]))

@@ -266,7 +266,7 @@ struct Workspace {
     double* p = nullptr;
     size_t n = 0;
 };
-std::mutex g_ws_mutex;
+std::recursive_mutex g_ws_mutex;   // a launcher's hold spans its own vlxmi_ket_workspace call
 std::map<std::pair<int, void*>, Workspace> g_ws;   // (device, stream) -> buffer
 }  // namespace
 
@@ -281,7 +281,7 @@ extern "C" int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out)
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    std::lock_guard<std::recursive_mutex> lock(g_ws_mutex);
     Workspace& w = g_ws[std::make_pair(dev, stream)];
     if (w.n < ndoubles) {
         if (w.p) {
@@ -303,9 +303,20 @@ extern "C" int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out)
     return VLXMI_OK;
 }
 
+// See vlxmi::WorkspaceHold.
+extern "C" void vlxmi_workspace_hold(int on)
+{
+    if (on)
+        g_ws_mutex.lock();
+    else
+        g_ws_mutex.unlock();
+}
+
 // As vlxmi_ket_workspace for launches that can do without: an error, with
 // nothing changed and no HIP error left behind, when the stream is being
-// captured or the memory is not to be had.
+// captured or the memory is not to be had.  The allocation is none of another
+// thread's capture's business (relaxed mode): these launchers allocated nothing
+// before they had a split, and ran beside a capture.
 extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out)
 {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -314,7 +325,10 @@ extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out)
         return VLXMI_ERR_ARG;
     }
     if (capturing != hipStreamCaptureStatusNone) return VLXMI_ERR_ARG;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
     const int rc = vlxmi_ket_workspace(ndoubles, stream, out);
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (rc > 0) (void)hipGetLastError();
     return rc;
 }
@@ -322,7 +336,7 @@ extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out)
 // Frees every ket-split workspace (after a device synchronization).
 extern "C" int vlxmi_release_workspaces(void)
 {
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    std::lock_guard<std::recursive_mutex> lock(g_ws_mutex);
     if (!g_ws.empty()) {
         hipError_t e = hipDeviceSynchronize();
         if (e != hipSuccess) return (int)e;

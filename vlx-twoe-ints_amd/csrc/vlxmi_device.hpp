@@ -52,8 +52,21 @@ extern "C" int vlxmi_validate_k_csr(uint32_t la, uint32_t lb, uint32_t count_a, 
 // Ket-split partial sums of the launchers (vlxmi_capi.cpp).
 extern "C" int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out);
 extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out);
+extern "C" void vlxmi_workspace_hold(int on);
 extern "C" int vlxmi_ket_split_reduce(const double* part, uint32_t nsplit, uint32_t count, double* out,
                                       void* stream);
+
+namespace vlxmi {
+// Held by a launcher from taking its workspace to enqueueing the reduction that
+// reads it: another thread on the same stream neither regrows the buffer nor
+// puts its own partial sums between the two launches.
+struct WorkspaceHold {
+    WorkspaceHold() { vlxmi_workspace_hold(1); }
+    ~WorkspaceHold() { vlxmi_workspace_hold(0); }
+    WorkspaceHold(const WorkspaceHold&) = delete;
+    WorkspaceHold& operator=(const WorkspaceHold&) = delete;
+};
+}  // namespace vlxmi
 
 #define VLX_BOYS_NCOL 16
 #define VLX_BOYS_NROW 2001
@@ -62,8 +75,6 @@ extern "C" int vlxmi_ket_split_reduce(const double* part, uint32_t nsplit, uint3
 #define VLX_BOYS_TMAX 40.0
 #define VLX_BOYS_CROWS 101
 #define VLX_BOYS_CDT 0.4
-#define VLX_BOYS_INV_CDT 2.5
-#define VLX_BOYS_CTERMS 12
 #define VLX_BOYS_LROWS 200
 #define VLX_BOYS_LCOLS 10
 #define VLX_BOYS_COARSE_OFF (VLX_BOYS_NROW * VLX_BOYS_NCOL)

@@ -75,14 +75,14 @@ ket_bounds_kernel(KetClasses K, const double* __restrict__ D, uint32_t n, double
     const vlxmi_ket_class& c = K.c[blockIdx.y];
     const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= c.nblk) return;
-    double top = 0.0;
+    unsigned long long top = 0;        // ordered as the values; a NaN leads its list
     for (uint32_t t = 0; t < c.nab; ++t) {
         const uint64_t e = b * c.nab + t;
         const double v = c.keep[e] ? D[(uint64_t)c.ao_first[e] * n + (uint64_t)c.ao_second[e]] : 0.0;
         mat_D[c.entry_offset + e] = v;
-        top = fmax(top, fabs(c.mat_Q[e] * v));
+        top = max(top, abs_bits(c.mat_Q[e] * v));
     }
-    beta[c.block_offset + b] = top;
+    beta[c.block_offset + b] = __longlong_as_double((long long)top);
 }
 
 // The ket copy of every list: block p of the output is block order[p] of the

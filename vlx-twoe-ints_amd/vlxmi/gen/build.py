@@ -105,9 +105,9 @@ def load_k_light():
 J_UNPACKED = ("ss", "sp")
 
 
-# gradient classes whose kernels run one pass per ket-first-index component
-# (emit_grad.grad_groups); the others run one pass.  Chosen from per-class
-# timings of both on lattice64.
+# recursion gradient classes whose kernels run more than one pass
+# (emit_grad.grad_groups), and the exchange classes with one-centre kernels;
+# chosen from per-class timings (the file's _doc)
 GRAD_PASSES_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "grad_passes.json")
 
 
@@ -239,8 +239,8 @@ SPLIT_SERIES = {"J": {"pddd": 7, "ddpd": 10, "dddd": 30},
 
 def splits_text():
     """Launchers named after the reference's split kernels: split 0 runs the
-    whole class (these kernels are split into component passes inside one
-    launch instead), splits 1..n-1 check their arguments and launch nothing,
+    whole class (these kernels run such classes as passes over Rys points
+    inside one launch instead), splits 1..n-1 check their arguments and launch nothing,
     so a host that launches the whole series into one buffer gets the class's
     result."""
     o = []

@@ -11,13 +11,16 @@ The bodies are this project's own design (see the module docstrings of
 J: one lane owns one bra primitive-pair block (all na*nb components); the
    wave walks the ket blocks in order, staging per-block records (eta, Q, QC,
    CD, S*D*w per component, |Q*D| per component, block bound) in LDS, one record
-   per lane; each lane evaluates the whole primitive quartet by straight-line
-   HGP code and digests every component with the reference's per-component
+   per lane; each lane evaluates the whole primitive quartet, by straight-line
+   HGP code (light classes) or as a sum over Rys points (rys.json), and digests every component with the reference's per-component
    screen |Q_ij Q_kl D_kl| > thr (as D_kl-weight select against the lane's
    per-component threshold thr/|Q_ij|).  Lanes leave the scan at the first ket
    block whose bound fails (blocks are sorted).  grid.y splits the ket list;
-   with more than one split the per-lane sums are added atomically.
-K: one workgroup (one wave) owns one (I,K) primitive block of the ik list;
+   the launcher's chunks write partial sums that one ordered reduction adds.
+   A tile of few bra blocks is packed: groups of lanes take different ket
+   records (pack_decls).
+K: one wavefront owns one (I,K) primitive block of the ik list (or, where the
+   list is short, a chunk of the block's ket tiles);
    lanes take partner blocks J of I, the wave walks the partner blocks L of K in
    order (LDS-staged records), each lane evaluates (IJ|KL) and digests with the
    reference's per-component screen |Q_ij Q_kl maxD_bd| > thr against D_AO
@@ -168,7 +171,10 @@ def rys_pass(la, lb, lc, ld, group, prefix, ind):
     """One pass: X{tab}_{tcd} = sum over the points of Ix Iy Iz for every bra
     component pair tab and the ket pairs of ``group``.  The points run in a
     loop that is not unrolled: one point's one-dimensional integrals are live
-    at a time and the kernel's code stays within the instruction cache."""
+    at a time and the kernel's code stays within the instruction cache.
+    FP64-issue bound; as the recursion, whose table of three-dimensional
+    intermediates was recomputed per pass or spilled, 48 atoms: K (pd|dd)
+    56.8 -> 10.7 ms, (sd|dd) 43.2 -> 7.8."""
     nb, nd = NC["spd"[lb]], NC["spd"[ld]]
     n = ryspts.nroots(la + lb + lc + ld)
     pt = RysPoint(prefix=prefix)
@@ -932,12 +938,14 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
              % (lc, ld, cd, cd, cd, cd, cd))
     o.append("        if (rc != 0) return rc;")
     o.append("    }")
-    o.append("    double* part = nullptr;")
     o.append("    if (ket_split > 1) {")
+    o.append("        vlxmi::WorkspaceHold hold;")
+    o.append("        double* part = nullptr;")
     o.append("        const int rc = vlxmi_ket_workspace((size_t)ket_split * %s_prim_pair_count_local, stream, &part);" % ab)
     o.append("        if (rc != 0) return rc;")
+    o.append("        return vlxmi_jpart_%s(%s, ket_split, part, stream);" % (name, ", ".join(args)))
     o.append("    }")
-    o.append("    return vlxmi_jpart_%s(%s, ket_split, part, stream);" % (name, ", ".join(args)))
+    o.append("    return vlxmi_jpart_%s(%s, ket_split, nullptr, stream);" % (name, ", ".join(args)))
     o.append("}")
     return "\n".join(o) + "\n"
 
@@ -957,12 +965,15 @@ def k_split_launch(name, ncomp, ket_count, out_count, max_d, grid, threads, args
     return ["    if (!(%s > 0.0)) return VLXMI_OK;" % max_d,
             "    const uint32_t tiles = (%s + %d) / %d, want = (%du + nblk - 1) / nblk;" % (ket_count, kt - 1, kt, 2048 if ncomp >= 27 else 512),
             "    const uint32_t split = want < tiles ? (want < 16 ? want : 16) : (tiles < 16 ? tiles : 16);",
-            "    double* part = nullptr;",
-            "    if (split > 1 && vlxmi_try_workspace((size_t)split * %s, stream, &part) == VLXMI_OK) {" % out_count,
-            "        hipLaunchKernelGGL(%s_ks, %s, dim3(%d), 0, (hipStream_t)stream, %s, part);" % (name, grid, threads, args),
-            "        const int rc = (int)hipGetLastError();",
-            "        if (rc != 0) return rc;",
-            "        return vlxmi_ket_split_reduce(part, split, %s, %s, stream);" % (out_count, out),
+            "    if (split > 1) {",
+            "        vlxmi::WorkspaceHold hold;",
+            "        double* part = nullptr;",
+            "        if (vlxmi_try_workspace((size_t)split * %s, stream, &part) == VLXMI_OK) {" % out_count,
+            "            hipLaunchKernelGGL(%s_ks, %s, dim3(%d), 0, (hipStream_t)stream, %s, part);" % (name, grid, threads, args),
+            "            const int rc = (int)hipGetLastError();",
+            "            if (rc != 0) return rc;",
+            "            return vlxmi_ket_split_reduce(part, split, %s, %s, stream);" % (out_count, out),
+            "        }",
             "    }"]
 
 

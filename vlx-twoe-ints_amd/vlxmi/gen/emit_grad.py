@@ -25,9 +25,10 @@ exchange energy gradients without new list data:
 Screening is the Fock kernels': a component quartet counts iff
 |Q_ij Q_kl D_kl| > thr (J, gen_coulomb.py:209-212) or |Q_ij Q_kl maxD_bd| > thr
 (K, gen_exchange.py:229-232).  The raised and lowered integrals come from the
-same concrete-component DAG as the Fock kernels (one more Boys order), in one
-pass or in one pass per ket-first-index component, a per-class choice
-(``grad_groups``, ``grad_passes.json``).  FP64 throughout.
+same concrete-component DAG as the Fock kernels (one more Boys order), or from
+Rys points (``rysdag.gradient_terms``) for the classes whose raised recursion
+does not fit the registers, a per-class choice (``rys.json``): FP64-issue bound,
+36 atoms: exchange (dd|dd) 259 -> 6.7 ms, (pd|dp) 143 -> 21.8.  FP64 throughout.
 """
 
 from __future__ import annotations
@@ -78,8 +79,8 @@ def grad_groups(la, lb, lc, ld, passes="one"):
     """The passes of a gradient kernel over the ket component pairs
     (t = ic * nd + id): "one" -- a single pass; "component" -- one pass per
     ket-first-index component ic (the recursion recomputed per pass, fewer
-    values live at a time); "pair" -- one pass per pair t.  Neither fits the registers for the p/d classes;
-    which runs faster is measured per class (``grad_passes.json``)."""
+    values live at a time); "pair" -- one pass per pair t.
+    Which runs faster is measured per class (``grad_passes.json``)."""
     nc, nd = (lc + 1) * (lc + 2) // 2, (ld + 1) * (ld + 2) // 2
     if passes == "component":
         return [list(range(i * nd, (i + 1) * nd)) for i in range(nc)]
@@ -287,6 +288,7 @@ def emit_jgrad(cls, passes="one", rys=None):
           % (lc, ld, cd, cd, cd, cd, cd),
           "        if (rc != 0) return rc;",
           "    }",
+          "    vlxmi::WorkspaceHold hold;",
           "    double* part = nullptr;",
           "    int rc = vlxmi_ket_workspace((size_t)ket_split * nbra * 6, stream, &part);",
           "    if (rc != 0) return rc;",
