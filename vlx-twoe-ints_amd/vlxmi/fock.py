@@ -218,16 +218,27 @@ class FockEngine:
     def cart_density(self, D_sph):
         return self._density(D_sph)[0]
 
+    def _kernel_density(self, Dc):
+        """``Dc`` as vlxmi_ket_bounds reads it, through a raw pointer: naos x naos
+        contiguous doubles on the engine's device."""
+        t, n = self.torch, self.naos
+        if Dc.dim() != 2 or Dc.shape[0] < n or Dc.shape[1] < n:
+            raise ValueError("Cartesian density must be at least %d x %d, got %s" % (n, n, tuple(Dc.shape)))
+        if Dc.device != self.T.device or Dc.is_complex():
+            raise ValueError("Cartesian density must be real and on %s, got %s on %s" % (self.T.device, Dc.dtype, Dc.device))
+        return Dc[:n, :n].to(t.float64).contiguous()
+
     def prepare_kets(self, Dc):
         """mat_D per J list and the ket-ordered copies (device); ``mat_D_bra``
-        keeps mat_D in the resident (bra) order."""
+        keeps mat_D in the resident (bra) order.  ``Dc``: a real matrix on the
+        engine's device whose leading naos x naos part is the Cartesian density."""
         t = self.torch
+        Dc = self._kernel_density(Dc)
         L, st, n = lib(), self.dev.stream_ptr(), self._ket_entries
         f64 = t.empty((4, n), dtype=t.float64, device=Dc.device)        # mat_D (bra order), then the ket copies
         ints = t.empty((2, n), dtype=t.int32, device=Dc.device)
         beta = t.empty(self._ket_blocks, dtype=t.float64, device=Dc.device)
         cls = type(self._ket_cls).from_buffer_copy(self._ket_cls)
-        Dc = Dc.contiguous()
         if n:
             check(L.vlxmi_ket_bounds(cls, len(cls), Dc.data_ptr(), self.naos, f64[0].data_ptr(), beta.data_ptr(), st), "ket_bounds")
             orders = []
