@@ -739,13 +739,16 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
         o.append("                    const double w = (%s_first_inds[f0 + t] != %s_second_inds[f0 + t]) ? 2.0 : 1.0;" % (cd, cd))
     else:
         o.append("                    const double w = 2.0;")
-    o.append("                    R[%d + t] = %s_pair_data[f0 + t] * Dkl * w;" % (KREC0, cd))
     o.append("                    const double qd = fabs(%s_mat_Q[f0 + t] * Dkl);" % cd)
+    # a component whose bound is NaN passes no screen: it takes the masks, and
+    # there is nothing to multiply the masked zero by
+    o.append("                    const double Sw = %s_pair_data[f0 + t] * Dkl * w;" % cd)
+    o.append("                    R[%d + t] = %s;" % (KREC0, "qd >= 0.0 ? Sw : 0.0" if whole else "Sw"))
     o.append("                    R[%d + NCD + t] = qd;" % KREC0)
     o.append("                    beta = fmax(beta, qd);")
     if whole:
         # a component whose density weight is zero adds nothing, masked or not
-        o.append("                    qmin = fmin(qmin, Dkl != 0.0 ? qd : qmin);")
+        o.append("                    qmin = fmin(qmin, Dkl != 0.0 ? fmax(qd, 0.0) : qmin);")
     o.append("                }")
     if whole:
         o.append("                R[%d] = qmin;" % (rec - 1))
@@ -852,7 +855,12 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("        const uint32_t e0 = bb * NAB;")
     o.append("        #pragma unroll")
     o.append("        for (int t = 0; t < NAB; ++t) {")
-    o.append("            const double v = %s_pair_data_local[e0 + t] * %s;" % (ab, "lacc[t * TILE_SIZE_J + lane]" if jlds else "acc[t]"))
+    accv = "lacc[t * TILE_SIZE_J + lane]" if jlds else "acc[t]"
+    if whole and not rys:
+        # nothing passes an infinite (or 0/0) threshold; the loop's masked zeros
+        # there are NaN if a ket density is infinite
+        accv = "(tau[t] < __builtin_inf() ? %s : 0.0)" % accv
+    o.append("            const double v = %s_pair_data_local[e0 + t] * %s;" % (ab, accv))
     if batched:
         o.append("            mat_J[e0 + t] += v;")
     else:
@@ -1215,12 +1223,13 @@ def emit_k(cls, mixed=False, batched=False, kt=None, layout="reg", dorder="jl", 
     o.append("                        #pragma unroll")
     o.append("                        for (int cdd = 0; cdd < ND; ++cdd) {")
     o.append("                            const uint32_t pos = displ_k[cc] + lp * ND + cdd;")
-    o.append("                            const double q = fabs(Q_K_%s[pos]);" % cd)
+    o.append("                            const double q = fabs(Q_K_%s[pos]), Sk = pair_data_K_%s[pos];" % (cd, cd))
     o.append("                            qk = fmax(qk, q);")
     if not heavy:
-        # a component whose factor is zero adds nothing, masked or not
-        o.append("                            if (pair_data_K_%s[pos] != 0.0) qmin = fmin(qmin, q);" % cd)
-    o.append("                            R[%d + cc * ND + cdd] = pair_data_K_%s[pos];" % (KREC0, cd))
+        # a component whose factor is zero adds nothing, masked or not; one whose
+        # bound is NaN passes no screen: masks, and nothing to multiply
+        o.append("                            if (Sk != 0.0) qmin = fmin(qmin, fmax(q, 0.0));")
+    o.append("                            R[%d + cc * ND + cdd] = %s;" % (KREC0, "Sk" if heavy else "q >= 0.0 ? Sk : 0.0"))
     o.append("                            R[%d + NCD + cc * ND + cdd] = q;" % KREC0)
     o.append("                        }")
     o.append("                    }")
