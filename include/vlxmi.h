@@ -66,8 +66,12 @@ int vlxmi_fill_zero(double* p, uint64_t n, void* stream);
  * (current device, stream) -- launches on one stream share it, other streams get
  * their own -- and then calls vlxmi_ket_split_reduce on the same stream.
  * vlxmi_ket_workspace returns (in *out) a buffer of at least ndoubles doubles,
- * growing it after synchronizing the stream; vlxmi_release_workspaces frees all
- * of them after a device synchronization. */
+ * growing it after synchronizing the stream; while the stream is being captured
+ * it allocates nothing: a large enough buffer belongs to the graph from then on
+ * (growth leaves it alone), else the call returns
+ * hipErrorStreamCaptureUnsupported and the launchers run unsplit.
+ * vlxmi_release_workspaces frees all of them, those of graphs and of the exchange
+ * launchers included, after a device synchronization. */
 int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out);
 int vlxmi_release_workspaces(void);
 

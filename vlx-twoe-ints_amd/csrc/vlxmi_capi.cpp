@@ -5,9 +5,6 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
-#include <map>
-#include <mutex>
-#include <utility>
 
 #include "vlxmi_device.hpp"
 
@@ -260,92 +257,6 @@ extern "C" int vlxmi_fill_zero(double* p, uint64_t n, void* stream)
 // is bit-reproducible) and carries about one rounding of the total instead of
 // one per chunk.
 // ---------------------------------------------------------------------------
-
-namespace {
-struct Workspace {
-    double* p = nullptr;
-    size_t n = 0;
-};
-std::recursive_mutex g_ws_mutex;   // a launcher's hold spans its own vlxmi_ket_workspace call
-std::map<std::pair<int, void*>, Workspace> g_ws;   // (device, stream) -> buffer
-}  // namespace
-
-// A device buffer of at least ndoubles doubles reserved for launches on
-// (current device, stream): launches on one stream run in order, so they can
-// share it; another stream gets its own.  Grown on demand (after synchronizing
-// the stream, whose earlier launches may still read the old buffer) and kept
-// until vlxmi_release_workspaces().
-extern "C" int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out)
-{
-    if (!out) return VLXMI_ERR_ARG;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return (int)e;
-    std::lock_guard<std::recursive_mutex> lock(g_ws_mutex);
-    Workspace& w = g_ws[std::make_pair(dev, stream)];
-    if (w.n < ndoubles) {
-        if (w.p) {
-            e = hipStreamSynchronize((hipStream_t)stream);
-            if (e != hipSuccess) return (int)e;
-            (void)hipFree(w.p);
-            w.p = nullptr;
-            w.n = 0;
-        }
-        const size_t n = ndoubles + ndoubles / 4;
-        e = hipMalloc((void**)&w.p, n * sizeof(double));
-        if (e != hipSuccess) {
-            w.p = nullptr;
-            return (int)e;
-        }
-        w.n = n;
-    }
-    *out = w.p;
-    return VLXMI_OK;
-}
-
-// See vlxmi::WorkspaceHold.
-extern "C" void vlxmi_workspace_hold(int on)
-{
-    if (on)
-        g_ws_mutex.lock();
-    else
-        g_ws_mutex.unlock();
-}
-
-// As vlxmi_ket_workspace for launches that can do without: an error, with
-// nothing changed and no HIP error left behind, when the stream is being
-// captured or the memory is not to be had.  The allocation is none of another
-// thread's capture's business (relaxed mode): these launchers allocated nothing
-// before they had a split, and ran beside a capture.
-extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out)
-{
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) {
-        (void)hipGetLastError();
-        return VLXMI_ERR_ARG;
-    }
-    if (capturing != hipStreamCaptureStatusNone) return VLXMI_ERR_ARG;
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    const int rc = vlxmi_ket_workspace(ndoubles, stream, out);
-    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (rc > 0) (void)hipGetLastError();
-    return rc;
-}
-
-// Frees every ket-split workspace (after a device synchronization).
-extern "C" int vlxmi_release_workspaces(void)
-{
-    std::lock_guard<std::recursive_mutex> lock(g_ws_mutex);
-    if (!g_ws.empty()) {
-        hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) return (int)e;
-    }
-    for (auto& kv : g_ws)
-        if (kv.second.p) (void)hipFree(kv.second.p);
-    g_ws.clear();
-    return VLXMI_OK;
-}
 
 __device__ __forceinline__ void neumaier_add(double& s, double& c, double x)
 {

@@ -49,7 +49,7 @@ extern "C" int vlxmi_validate_ik_list(uint32_t la, uint32_t lc, const uint32_t* 
 extern "C" int vlxmi_validate_k_csr(uint32_t la, uint32_t lb, uint32_t count_a, const uint32_t* displs,
                                     const uint32_t* counts, const double* Q, const uint32_t* D_inds, void* stream);
 
-// Ket-split partial sums of the launchers (vlxmi_capi.cpp).
+// Ket-split partial sums of the launchers (vlxmi_workspace.cpp, vlxmi_capi.cpp).
 extern "C" int vlxmi_ket_workspace(size_t ndoubles, void* stream, double** out);
 extern "C" int vlxmi_try_workspace(size_t ndoubles, void* stream, double** out);
 extern "C" void vlxmi_workspace_hold(int on);

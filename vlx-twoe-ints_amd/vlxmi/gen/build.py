@@ -586,7 +586,8 @@ def _build(jobs=None, force=False, only=None, verbose=True):
         f.write(device_header_text())
     todo = []
     objs = []
-    hand = ["vlxmi_capi.cpp", "vlxmi_noalloc.cpp", "vlxmi_lists.cpp", "vlxmi_pairs.cpp", "vlxmi_prep.cpp"]
+    hand = ["vlxmi_capi.cpp", "vlxmi_noalloc.cpp", "vlxmi_lists.cpp", "vlxmi_pairs.cpp", "vlxmi_prep.cpp",
+            "vlxmi_workspace.cpp"]
     flag_key = " ".join(FLAGS)
     dev_hdr = open(os.path.join(CSRC, "vlxmi_device.hpp")).read() + open(os.path.join(CSRC, "vlxmi_status.h")).read()
     prep_hdr = open(os.path.join(ROOT, "include", "vlxmi_prep.h")).read()

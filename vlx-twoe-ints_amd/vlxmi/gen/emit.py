@@ -950,10 +950,10 @@ def emit_j(cls, mixed=False, batched=False, kt=None, layout="reg", lds_boys=Fals
     o.append("        vlxmi::WorkspaceHold hold;")
     o.append("        double* part = nullptr;")
     o.append("        const int rc = vlxmi_ket_workspace((size_t)ket_split * %s_prim_pair_count_local, stream, &part);" % ab)
-    o.append("        if (rc != 0) return rc;")
-    o.append("        return vlxmi_jpart_%s(%s, ket_split, part, stream);" % (name, ", ".join(args)))
+    o.append("        if (rc == VLXMI_OK) return vlxmi_jpart_%s(%s, ket_split, part, stream);" % (name, ", ".join(args)))
+    o.append("        if (rc != (int)hipErrorStreamCaptureUnsupported) return rc;   // a capture without the memory: unsplit")
     o.append("    }")
-    o.append("    return vlxmi_jpart_%s(%s, ket_split, nullptr, stream);" % (name, ", ".join(args)))
+    o.append("    return vlxmi_jpart_%s(%s, 1, nullptr, stream);" % (name, ", ".join(args)))
     o.append("}")
     return "\n".join(o) + "\n"
 

@@ -291,6 +291,10 @@ def emit_jgrad(cls, passes="one", rys=None):
           "    vlxmi::WorkspaceHold hold;",
           "    double* part = nullptr;",
           "    int rc = vlxmi_ket_workspace((size_t)ket_split * nbra * 6, stream, &part);",
+          "    if (rc == (int)hipErrorStreamCaptureUnsupported && ket_split > 1) {   // a capture without the memory: unsplit",
+          "        ket_split = 1;",
+          "        rc = vlxmi_ket_workspace((size_t)nbra * 6, stream, &part);",
+          "    }",
           "    if (rc != 0) return rc;",
           "    hipLaunchKernelGGL(%s, dim3((nbra + 63) / 64, ket_split), dim3(64), 0, (hipStream_t)stream, %s);"
           % (name, ", ".join(["part"] + args[1:])),
