@@ -28,10 +28,11 @@
 // single-precision hardware exponential is accurate enough for it.
 //
 // Coarse rows (after the fine table, VLX_BOYS_CROWS rows of VLX_BOYS_NCOL
-// doubles): F_0..F_15 at T_k = k * VLX_BOYS_CDT; kept in the table's layout, no
-// kernel reads them.  Kernels of the light classes make their own rows in LDS
-// from every tenth fine row, once per workgroup (boys_lds_fill), and evaluate
-// F_L from there: no global gather per quartet.
+// doubles): F_0..F_15 at T_k = k * VLX_BOYS_CDT.  No kernel reads them; they
+// stay because the layout is public (callers size and fill their tables with
+// vlxmi_boys_table_size / _fill, and check it).  Kernels of the light classes
+// make their own rows in LDS from every tenth fine row, once per workgroup
+// (boys_lds_fill), and evaluate F_L from there: no global gather per quartet.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -177,11 +178,13 @@ __device__ __forceinline__ void boys(double T, const double* __restrict__ table,
 }
 
 // The LDS rows of order L: row k covers T in [k/5, (k+1)/5), T_k = k/5 + 1/10 (a
-// fine row of the table): columns 0..7 the degree-7 polynomial of F_L in
-// x = 10 (T - T_k), |x| <= 1, column 8 exp(-T_k).  The polynomial is the
+// fine row of the table): columns 0..8 the degree-8 polynomial of F_L in
+// x = 10 (T - T_k), |x| <= 1, column 9 exp(-T_k).  The polynomial is the
 // degree-10 Taylor expansion F_L = sum_j F_{L+j}(T_k) (-x/10)^j / j! with its
-// three highest powers replaced by their Chebyshev economisation (error below
-// 0.1^8 / (8! 2^7) F_{L+8} < 2e-15 F_{L+8}(T_k), at most 7e-16 F_L for L <= 4).
+// two highest powers replaced by their Chebyshev economisation (error below
+// 0.1^9 / (9! 2^8) F_{L+9} = 1e-17 F_{L+9}); against 113-bit arithmetic F_L is
+// within 4.2e-16 relative for L <= 4 (degree 7: 9.7e-16 at one instruction
+// less a quartet).
 // Ten doubles a row: 16-byte reads of random rows spread over all LDS banks.
 // Every thread of the workgroup calls it; the caller synchronises afterwards.
 template <int L>
@@ -205,13 +208,9 @@ __device__ __forceinline__ void boys_lds_fill(const double* __restrict__ table, 
         c[5] -= c[9] * (432.0 / 256.0);
         c[3] += c[9] * (120.0 / 256.0);
         c[1] -= c[9] * (9.0 / 256.0);
-        c[6] += c[8] * (256.0 / 128.0);
-        c[4] -= c[8] * (160.0 / 128.0);
-        c[2] += c[8] * (32.0 / 128.0);
-        c[0] -= c[8] * (1.0 / 128.0);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) lt[r * VLX_BOYS_LCOLS + j] = c[j];
-        lt[r * VLX_BOYS_LCOLS + 8] = row[15];
+        for (int j = 0; j < 9; ++j) lt[r * VLX_BOYS_LCOLS + j] = c[j];
+        lt[r * VLX_BOYS_LCOLS + 9] = row[15];
     }
 }
 
@@ -226,9 +225,9 @@ __device__ __forceinline__ void boys_lds(double T, const double* lt, double* F)
         const int k = (int)(T * 5.0);
         const double x = fma(T, 10.0, -(double)(2 * k + 1));
         const double* row = lt + k * VLX_BOYS_LCOLS;
-        double s = row[7];
+        double s = row[8];
 #pragma unroll
-        for (int j = 6; j >= 0; --j) s = fma(s, x, row[j]);
+        for (int j = 7; j >= 0; --j) s = fma(s, x, row[j]);
         F[L] = s;
         if (L > 0) {
             constexpr double t9 = -1e-9 / 362880.0, t10 = 1e-10 / 3628800.0;
@@ -241,7 +240,7 @@ __device__ __forceinline__ void boys_lds(double T, const double* lt, double* F)
             e = fma(e, x, 1e-2 / 2.0 - t10 * (50.0 / 512.0));
             e = fma(e, x, -1e-1 - t9 * (9.0 / 256.0));
             e = fma(e, x, 1.0 + t10 * (1.0 / 512.0));
-            const double et = row[8] * e;
+            const double et = row[9] * e;
             const double T2 = 2.0 * T;
 #pragma unroll
             for (int m = L - 1; m >= 0; --m) F[m] = fma(T2, F[m + 1], et) * (1.0 / (2.0 * m + 1.0));
@@ -251,7 +250,8 @@ __device__ __forceinline__ void boys_lds(double T, const double* lt, double* F)
         F[0] = (0.5 * 1.77245385090551602730) * y;
         if (L > 0) {
             const double et = (double)__expf(-(float)T);
-            const double h = 0.5 * (y * y);
+            // 1/T as y^2 with y's rounding taken out: F_m multiplies it m times
+            const double y2 = y * y, h = 0.5 * fma(y2, fma(-T, y2, 1.0), y2);
 #pragma unroll
             for (int m = 0; m < L; ++m) F[m + 1] = ((2.0 * m + 1.0) * F[m] - et) * h;
         }
