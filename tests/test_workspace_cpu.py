@@ -92,6 +92,7 @@ extern "C" const char* model_log(void) { static std::string out; out = g_log; g_
 """
 
 S1, S2 = 0x1000, 0x2000
+UNIT = 1 << 18                # the smallest buffer, in doubles
 
 
 @pytest.fixture(scope="module")
@@ -122,7 +123,7 @@ def ws(so, tmp_path):
 
 def _take(L, n, stream=S1, exchange=False):
     p = C.c_void_p()
-    rc = (L.vlxmi_try_workspace if exchange else L.vlxmi_ket_workspace)(n, stream, C.byref(p))
+    rc = (L.vlxmi_try_workspace if exchange else L.vlxmi_ket_workspace)(int(n * UNIT), stream, C.byref(p))
     return rc, p.value
 
 
@@ -170,7 +171,7 @@ def test_a_graphs_buffer_outlives_growth(ws):
         n = int(n * 1.3)
     rc, last = _take(ws, 100 * n)
     assert rc == OK and all(ws.model_live(p) for p, _ in kept)
-    assert ws.model_used() < 2 * 8 * 125 * n + 8
+    assert ws.model_used() < 2 * 8 * UNIT * 125 * n
     _take(ws, 200 * n)                                     # not a graph's: freed
     assert not ws.model_live(last) and all(ws.model_live(p) for p, _ in kept)
     assert ws.vlxmi_release_workspaces() == OK and ws.model_used() == 0
@@ -187,12 +188,13 @@ def test_out_of_memory(ws):
     """An exchange launch keeps its old buffer and leaves no error behind; a
     Coulomb launch gives its old buffer up for the new one."""
     a, b = _take(ws, 80)[1], _take(ws, 80, exchange=True)[1]
-    ws.model_room(8 * 250)
+    ws.model_room(8 * UNIT * 250)
     assert _take(ws, 120, exchange=True)[0] == OOM and ws.model_live(b) and ws.model_last() == 0
     assert _take(ws, 80, exchange=True) == (OK, b)
     ws.model_log()
     rc, c = _take(ws, 110)
     assert rc == OK and not ws.model_live(a) and ws.model_log() == b"sfm" and ws.model_last() == 0
+    assert ws.model_used() == 8 * UNIT * (100 + 137.5)
     assert _take(ws, 1000)[0] == OOM
     ws.model_room(1 << 40)
     assert _take(ws, 1000)[0] == OK
@@ -205,3 +207,14 @@ def test_failed_synchronisation_leaks_nothing(ws):
     assert _take(ws, 800)[0] == SYNC_FAILED and ws.model_live(a) and ws.model_used() == used
     ws.model_sync_fails(0)
     assert _take(ws, 80) == (OK, a)
+
+
+def test_first_buffer_holds_what_small_molecules_ask_for(ws):
+    """One allocation for all requests up to 2 MiB; only what was asked for when
+    no more is to be had."""
+    for n in (1, 50, 3000, 1 << 18):
+        assert _take(ws, n / UNIT, exchange=True)[0] == OK
+    assert ws.model_log() == b"m" and ws.model_used() == 1 << 21
+    ws.model_room((1 << 21) + 8000)
+    assert _take(ws, 1000 / UNIT, S2)[0] == OK and ws.model_used() == (1 << 21) + 8000
+    assert ws.model_last() == 0

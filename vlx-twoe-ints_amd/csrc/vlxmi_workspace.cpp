@@ -52,16 +52,41 @@ struct RelaxedCapture {
     }
 };
 
+// A new buffer holds at least 2 MiB, as much as any exchange launch asks for (its
+// chunks times blocks are fewer than 4096, at most 36 sums each): growing class
+// by class, each time with a synchronisation, an allocation and a free, lengthened
+// the first build on a stream.
+constexpr size_t MIN_DOUBLES = (size_t)1 << 18;
+
+// A buffer of n doubles, with room to spare if it is to be had (``spare``).
+hipError_t allocate(size_t n, size_t spare, double** p, size_t* got)
+{
+    hipError_t e = hipSuccess;
+    for (size_t want : {spare, n}) {
+        e = hipMalloc((void**)p, want * sizeof(double));
+        if (e == hipSuccess) {
+            *got = want;
+            break;
+        }
+        if (want != n) (void)hipGetLastError();
+    }
+    return e;
+}
+
 // Grows w to n doubles; the old buffer stays as it was on failure, unless
 // ``need`` and only its memory makes room for the new one.
 hipError_t grow(Workspace& w, size_t n, hipStream_t stream, bool need)
 {
     RelaxedCapture relaxed;
     if (w.in_graph) w.retired.reserve(w.retired.size() + 1);
-    size_t want = n + n / 4;
-    if (w.in_graph && want < 2 * w.n) want = 2 * w.n;
+    size_t spare = n + n / 4, least = n, got = 0;
+    if (spare < MIN_DOUBLES) spare = MIN_DOUBLES;
+    if (w.in_graph) {
+        if (spare < 2 * w.n) spare = 2 * w.n;
+        least = spare;
+    }
     double* p = nullptr;
-    hipError_t e = hipMalloc((void**)&p, want * sizeof(double));
+    hipError_t e = allocate(least, spare, &p, &got);
     if (e != hipSuccess && (!need || !w.p || w.in_graph)) return e;
     if (w.p && w.in_graph) {
         w.retired.push_back(w.p);
@@ -77,12 +102,12 @@ hipError_t grow(Workspace& w, size_t n, hipStream_t stream, bool need)
             (void)hipGetLastError();
             w.p = nullptr;
             w.n = 0;
-            e = hipMalloc((void**)&p, want * sizeof(double));
+            e = allocate(least, spare, &p, &got);
             if (e != hipSuccess) return e;
         }
     }
     w.p = p;
-    w.n = want;
+    w.n = got;
     w.in_graph = false;
     return hipSuccess;
 }
