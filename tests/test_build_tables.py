@@ -137,6 +137,16 @@ def test_mixed_policy_table():
         policy.use_mixed("K", "ssss", "mixed", "some")
 
 
+def test_mixed_policy_takes_no_precision_from_a_class():
+    """By default only classes of the table's first version may run FP32 in mixed
+    precision: a class whose quartets were FP64 there stays FP64."""
+    from vlxmi import policy
+    first = {"J": "ddpp ddsd ddsp pdpp pdsd ppdd pppd ppsp sddd sdpd spdd sppp spsd", "K": "dpdd dpdp dsdd pdpd ppdp pppd psdd spdd"}
+    tab = policy.mixed_classes()
+    for kind in ("J", "K"):
+        assert tab[kind] <= set(first[kind].split()), kind
+
+
 def test_mixed_fp32_passes():
     """The FP32 part of a mixed kernel runs its own (never more) passes:
     FP32 intermediates take half the registers of FP64 ones.  A heavy exchange

@@ -4,10 +4,10 @@ gfx950 issues FP32 VALU instructions at the FP64 rate when packed FP32 is not
 used (the library is compiled without it), so running a class's VRR/HRR in FP32
 only pays where halving the recursion's registers removes spills; in the light
 classes the conversions make the ``_mixed`` kernel slower than the FP64 one.
-``gen/mixed_classes.json`` lists the classes whose ``_mixed`` kernel measured
-at least 3% faster than their FP64 kernel on lattice64; with the "measured"
-policy the engines launch the ``_mixed`` kernel for those classes and the FP64
-kernel for every other class, with policy "all" every class runs ``_mixed``.
+``gen/mixed_classes.json`` lists the classes that run it (its ``_doc`` has the
+timings on a 48-atom s/p/d lattice); with the "measured" policy the engines
+launch the ``_mixed`` kernel for those classes and the FP64 kernel for every
+other class, with policy "all" every class runs ``_mixed``.
 Either way no quartet above the FP32 bound is evaluated in FP32.
 """
 
