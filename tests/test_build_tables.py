@@ -50,7 +50,7 @@ def test_tile_table_entries():
 
 def test_sources_use_table_values():
     """Kernels take their ket tile from the tile table, except those that keep
-    the coarse Boys rows in LDS (a fixed 16-record tile)."""
+    Boys rows in LDS (a fixed 16-record tile)."""
     tiles = B.load_tiles()
     blds = B.load_boys_lds()
     srcs = B.sources()
@@ -170,26 +170,24 @@ def test_mixed_fp32_passes():
 def test_gradient_layout_table():
     """Every gradient class named in grad_passes.json has a known layout, and
     the generated sources follow it: Coulomb classes listed run one pass per
-    ket-first-index component or per ket component pair; exchange classes
-    split by centre have an _A and a _C kernel, launched one after the other
-    by the class launcher, each with one pass, one per ket-first-index
-    component or one per ket component pair."""
+    ket-first-index component or per ket component pair, exchange classes one
+    per ket-first-index component; the exchange classes under "centres" have an
+    _A and a _C kernel beside the class's own, the only one the launcher runs."""
     from vlxmi.gen import emit_grad
     gp = B.load_grad_passes()
     assert set(gp["J"].values()) <= {"component", "pair"} and gp["J"]
-    assert set(gp["K"].values()) <= {"component", "split_one", "split_component", "split_pair"} and gp["K"]
-    assert set(gp["J"]) <= {ab + cd for ab, cd in j_classes()} and set(gp["K"]) <= set(k_classes())
+    assert set(gp["K"].values()) <= {"component"} and gp["K"]
+    assert set(gp["J"]) <= {ab + cd for ab, cd in j_classes()} and set(gp["K"]) | gp["centres"] <= set(k_classes())
     srcs = B.sources()
+    for cls in k_classes():
+        s, name = srcs["kg_%s.hip" % cls], "computeExchangeGradient" + cls.upper()
+        for suffix in ("_A", "_C"):
+            assert ("%s%s(" % (name, suffix) in s) == (cls in gp["centres"]), cls
+            assert "hipLaunchKernelGGL(%s%s," % (name, suffix) not in s
+        assert s.count("hipLaunchKernelGGL(%s," % name) == 1 and s.count("hipLaunchKernelGGL(%s_ks," % name) == 1
     for cls, v in gp["K"].items():
-        passes, split = B.grad_k_layout(gp, cls)
-        s = srcs["kg_%s.hip" % cls]
-        name = "computeExchangeGradient" + cls.upper()
-        if split:
-            assert (name + "_A(") in s and (name + "_C(") in s
-            assert s.count("hipLaunchKernelGGL(%s_" % name) == 2
-        nc, nd = [(emit.LV[x] + 1) * (emit.LV[x] + 2) // 2 for x in cls[2:]]
-        assert len(emit_grad.grad_groups(*[emit.LV[x] for x in cls], passes)) == \
-            {"component": nc, "pair": nc * nd, "one": 1}[passes]
+        nc = (emit.LV[cls[2]] + 1) * (emit.LV[cls[2]] + 2) // 2
+        assert len(emit_grad.grad_groups(*[emit.LV[x] for x in cls], v)) == nc
     for cls, v in gp["J"].items():
         assert "computeCoulombGradient" + cls.upper() in srcs["jg_%s.hip" % cls]
         nc, nd = [(emit.LV[x] + 1) * (emit.LV[x] + 2) // 2 for x in cls[2:]]

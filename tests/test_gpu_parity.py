@@ -46,7 +46,7 @@ def test_boys_device(dev):
         rel = np.max(np.abs(F - ref) / np.abs(ref))
         assert rel < 1e-14, (L, rel)
         if L <= 4:
-            # the coarse rows in LDS (12-term Taylor) that some light-class kernels use
+            # the polynomial rows in LDS that the light-class kernels use
             Fc = dev.boys_eval(T, L, coarse=True)
             relc = np.max(np.abs(Fc - ref) / np.abs(ref))
             assert relc < 1e-14, (L, "coarse", relc)

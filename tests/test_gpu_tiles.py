@@ -53,9 +53,9 @@ def test_tiles_against_oracle(dev, n):
 
 @pytest.mark.parametrize("n", [12, 13, 16, 17, 24, 25, 32, 33, 48, 49, 64, 65])
 def test_tiles_sum_rule(dev, n):
-    """Lists of n partners against the same molecule's kernels run one (I,K)
-    block / one bra block at a time (a tile of one block each): sums of the
-    same terms in another order, at most 1e4 of them."""
+    """J of lists of n blocks against the same kernels on one bra block at a time
+    (a tile of one block): sums of the same terms in another order, at most 1e4
+    of them.  K of diagonal (I,I) blocks from both ends of the quartet."""
     from vlxmi.fock import FockEngine
     print("case: chain of %d atoms, sliced" % n, flush=True)
     mol, D = _chain(n)
@@ -70,7 +70,7 @@ def test_tiles_sum_rule(dev, n):
             assert np.abs(one - whole[b * nab:(b + 1) * nab]).max() <= 1e-12 * max(1.0, np.abs(whole).max())
     # K: the sum over the partners of an (I,K) block is symmetric in which side's
     # list is walked by lanes: (ab|cd) with I, K exchanged is the class (cd|ab)
-    for cls, other in (("ssss", "ssss"), ("spsd", "sdsp"), ("pppp", "pppp"), ("dsdp", "dpds")):
+    for cls, other in (("spsd", "sdsp"), ("pppp", "pppp"), ("dsdp", "dpds")):
         ac = cls[0] + cls[2]
         x = eng.run_K(Dc, classes=[cls], maxD=maxD)[ac].cpu().numpy()
         y = eng.run_K(Dc, classes=[other], maxD=maxD)[ac].cpu().numpy()
@@ -100,49 +100,153 @@ def test_gradient_tiles_against_oracle(dev, n):
                 assert np.abs(got[k].cpu().numpy() - ref[k]).max() <= 1e-11 * scale, k
 
 
-def test_exchange_split_under_capture(dev):
+@pytest.mark.parametrize("n", [13, 17, 25, 33])
+@pytest.mark.parametrize("cls", ["ssss", "ssps", "sppp", "pppp", "sdpd", "pddd"])
+def test_exchange_tiles_against_oracle(dev, cls, n):
+    """Partner counts on both sides of the narrowing step, with the launch split
+    where it splits: sampled (I,K) blocks of the whole launch against the oracle."""
+    from vlxmi.fock import FockEngine
+    from vlxmi.pairs import NCART, LVAL
+    print("case: chain of %d atoms, K %s" % (n, cls), flush=True)
+    mol, D = _chain(n)
+    eng = FockEngine(mol, dev=dev)
+    Dc = eng.cart_density(D)
+    ac = cls[0] + cls[2]
+    got = eng.run_K(Dc, classes=[cls])[ac].cpu().numpy()
+    nblk = eng.fl.iklists[ac].nblk
+    sel = np.unique([0, 1, nblk // 3, nblk // 2, nblk - 2, nblk - 1]).astype(np.uint32)
+    ref = U.oracle_matK(eng.fl, U.cart_density(mol, D), "component", ik_blocks=sel, classes=[cls])[ac]
+    nac = NCART[LVAL[cls[0]]] * NCART[LVAL[cls[2]]]
+    e = (sel[:, None].astype(np.int64) * nac + np.arange(nac)).ravel()
+    assert np.abs(ref[e]).max() > 0
+    assert np.abs(got[e] - ref[e]).max() <= 1e-11 * max(1.0, np.abs(ref[e]).max())
+
+
+def _mixed_run(eng, thr32, run):
+    """(FP64 result, mixed result, FP64 and FP32 quartets of the latter)."""
+    ref = run().cpu().numpy()
+    eng.precision, eng.mixed_policy, eng.fp32_threshold = "mixed", "all", thr32
+    eng.reset_counts()
+    got = run().cpu().numpy()
+    counts = eng.quartet_counts()
+    eng.precision = "fp64"
+    return ref, got, counts
+
+
+# an FP32 recursion's result carries at most some 64 roundings of the bound its
+# quartet was let through by (below the threshold)
+FP32_QUARTET = 64 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n", [5, 13, 17, 25, 33])
+def test_mixed_tiles_coulomb(dev, n):
+    """Packed bra tiles that change from FP64 to FP32 within a ket tile: every
+    quartet above the screen is evaluated once, none above the FP32 bound in
+    FP32, and the sums differ by what FP32 leaves out."""
+    from vlxmi import flops
+    from vlxmi.fock import FockEngine
+    print("case: chain of %d atoms, mixed J" % n, flush=True)
+    mol, D = _chain(n)
+    eng = FockEngine(mol, dev=dev)
+    Dc, Dn = eng.cart_density(D), U.cart_density(mol, D)
+    kets = eng.prepare_kets(Dc)
+    for ab, cd in (("pp", "sp"), ("pp", "pp"), ("pd", "ss"), ("pd", "dd")):
+        bra, ket = eng.fl.jlists[ab], eng.fl.jlists[cd]
+        beta = np.abs(ket.mat_Q * ket.mat_D(Dn)).reshape(ket.nblk, -1).max(axis=1)
+        thr32 = float(np.median(np.outer(bra.qmax_blk, beta)))
+        ref, got, (n64, n32) = _mixed_run(eng, thr32, lambda: eng.run_J(Dc, kets=kets, classes=[(ab, cd)])[ab])
+        assert n64 + n32 == flops.count_j(eng.fl, Dn, ab, cd) and n32 > 0, (ab, cd)
+        thr, eng.fl.thr = eng.fl.thr, thr32
+        assert n64 >= flops.count_j(eng.fl, Dn, ab, cd)
+        eng.fl.thr = thr
+        assert 0 < np.abs(got - ref).max() <= FP32_QUARTET * 2 * ket.count * thr32, (ab, cd)
+
+
+@pytest.mark.parametrize("n", [5, 13, 17, 25, 33])
+def test_mixed_tiles_exchange(dev, n):
+    """As test_mixed_tiles_coulomb for packed partner tiles."""
+    from vlxmi.fock import FockEngine
+    print("case: chain of %d atoms, mixed K" % n, flush=True)
+    mol, D = _chain(n)
+    eng = FockEngine(mol, dev=dev)
+    Dc = eng.cart_density(D)
+    maxD = eng.max_D(Dc)
+    for cls in ("ssps", "ppps", "sppp", "ppdp", "pddd"):
+        A, C = eng.fl.kcsr[cls[:2]], eng.fl.kcsr[cls[2:]]
+        mx = maxD[cls[1] + cls[3]]
+        thr32 = float(A.blk_max.max() * np.median(C.blk_max) * mx)      # every tile changes half-way
+        ref, got, (n64, n32) = _mixed_run(eng, thr32, lambda: eng.run_K(Dc, classes=[cls], maxD=maxD)[cls[0] + cls[2]])
+        assert n64 + n32 == eng.count_k_quartets(cls, mx), cls
+        assert n32 > 0 or n < 8, cls                     # up to 8 records are one step of 8 lane groups
+        thr, eng.thr = eng.thr, thr32
+        assert n64 >= eng.count_k_quartets(cls, mx)
+        eng.thr = thr
+        terms = A.Q.size // eng.fl.prims[0].count * (C.Q.size // eng.fl.prims[0].count)
+        assert np.abs(got - ref).max() <= FP32_QUARTET * terms * thr32, cls
+
+
+@pytest.fixture(scope="module")
+def split():
+    """The number of chunks an exchange launch of an engine takes, by the rule in
+    the launcher's source."""
+    import re
+    from vlxmi.gen import build
+    src = build.sources()
+
+    def chunks(eng, cls):
+        m = re.search(r"tiles = \((\w)_prim_count \+ \d+\) / (\d+), want = \((\d+)u", src["k_%s.hip" % cls])
+        nblk = eng.ik[cls[0] + cls[2]]["nblk"]
+        tiles = -(-eng.prim_count["spd".index(m.group(1))] // int(m.group(2)))
+        return min(tiles, -(-int(m.group(3)) // nblk), 16)
+    return chunks
+
+
+def test_exchange_split_under_capture(dev, split):
     """An exchange launch over few blocks splits its partners among wavefronts
     (partial sums in the library's workspace); while a stream is captured it
     stays unsplit, and the graph gives the same sums on every replay."""
     from vlxmi.fock import FockEngine
     print("case: exchange launches in a graph", flush=True)
     t = dev.torch
-    mol, D = _chain(12)
+    mol, D = _chain(17)
     eng = FockEngine(mol, dev=dev)
     Dc = eng.cart_density(D)
     maxD = eng.max_D(Dc)
     for cls in ("ssss", "dpds", "pddd"):
+        assert split(eng, cls) > 1
         ref = eng.run_K(Dc, classes=[cls], maxD=maxD)[cls[0] + cls[2]].clone()
         s = t.cuda.Stream(device=dev.device)
         s.wait_stream(t.cuda.current_stream(dev.device))
         g = t.cuda.CUDAGraph()
         with t.cuda.stream(s):
-            eng.run_K(Dc, classes=[cls], maxD=maxD)
+            eng.run_K(Dc, classes=[cls], maxD=maxD)          # the capturing stream has a workspace
         t.cuda.synchronize()
-        with t.cuda.graph(g):
+        with t.cuda.graph(g, stream=s):
             out = eng.run_K(Dc, classes=[cls], maxD=maxD)[cls[0] + cls[2]]
         for _ in range(3):
             g.replay()
             t.cuda.synchronize()
             assert (out - ref).abs().max() <= 1e-12 * max(1.0, float(ref.abs().max()))
-            eng.run_K(Dc, classes=[cls], maxD=maxD)
+            assert t.equal(eng.run_K(Dc, classes=[cls], maxD=maxD)[cls[0] + cls[2]], ref)
 
 
-def test_exchange_split_two_threads_one_stream(dev):
+def test_exchange_split_two_threads_one_stream(dev, split):
     """Two threads launch split exchange classes of different sizes on one
     stream: each gets the sums it gets alone, bit for bit (a launch and its
-    reduction hold the stream's workspace together)."""
+    reduction hold the stream's workspace together; every launch of both threads
+    uses it)."""
     import threading
     from vlxmi.fock import FockEngine
     print("case: two threads, one stream", flush=True)
     t = dev.torch
     work = []
-    for n in (9, 17):
+    classes = ("ssss", "dpds", "pddd", "sdpd")
+    for n in (17, 31):
         mol, D = _chain(n)
         eng = FockEngine(mol, dev=dev)
+        assert all(split(eng, c) > 1 for c in classes)
         Dc = eng.cart_density(D)
         work.append((eng, Dc, eng.max_D(Dc)))
-    classes = ("ssss", "dpds", "pddd", "sdpd")
 
     def run(w):
         eng, Dc, maxD = w
@@ -153,7 +257,7 @@ def test_exchange_split_two_threads_one_stream(dev):
     got = [[], []]
 
     def loop(i):
-        for _ in range(6):
+        for _ in range(20):
             got[i].append(run(work[i]))
 
     ts = [threading.Thread(target=loop, args=(i,)) for i in range(2)]
@@ -164,5 +268,5 @@ def test_exchange_split_two_threads_one_stream(dev):
     assert not any(x.is_alive() for x in ts)
     t.cuda.synchronize()
     for i in range(2):
-        assert len(got[i]) == 6
+        assert len(got[i]) == 20
         assert all(t.equal(a, b) for r in got[i] for a, b in zip(r, alone[i]))

@@ -111,12 +111,6 @@ J_UNPACKED = ("ss", "sp")
 GRAD_PASSES_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "grad_passes.json")
 
 
-def grad_k_layout(gp, cls):
-    """(passes, split) of the exchange-gradient recursion of ``cls``; no class
-    is split by centre any more (the second value is always False)."""
-    return gp["K"].get(cls, "one"), False
-
-
 def load_grad_passes():
     """{"J": {class: passes}, "K": {class: passes}, "centres": classes with
     one-centre kernels beside the class's own}; absent classes run one pass."""
@@ -219,7 +213,7 @@ def sources(tiles=None, layouts=None):
     for cls in k_classes():
         r = rys["KG"].get(cls)
         out["kg_%s.hip" % cls] = rys_inc(cls, 1, r) + inc + emit_grad.emit_kgrad(
-            cls, passes=grad_k_layout(gp, cls)[0], rys=r, centres=cls in gp["centres"])
+            cls, passes=gp["K"].get(cls, "one"), rys=r, centres=cls in gp["centres"])
     for n in range(1, ryspts.NMAX + 1):
         out["rys_table_%d.h" % n] = ryspts.header_text(n)
     for pc in PAIR_CLASSES:
