@@ -20,7 +20,7 @@ def eng(monkeypatch):
     e = fock.FockEngine.__new__(fock.FockEngine)
     e.torch, e.naos, e.T = torch, N, torch.eye(N, dtype=torch.float64)
     e.dev = types.SimpleNamespace(device=torch.device("cpu"), stream_ptr=lambda: 0)
-    e._ket_cls, e._ket_entries, e._ket_blocks, e.jl = (fock.KetClass * 0)(), 0, 0, {}
+    e.jl = {}
     monkeypatch.setattr(fock, "lib", lambda: None)
     return e
 
@@ -41,3 +41,17 @@ def test_converted_to_contiguous_doubles(eng):
 def test_refused(eng, bad):
     with pytest.raises(ValueError):
         eng.prepare_kets(bad)
+
+
+def test_lists_are_the_ones_in_place(eng):
+    """A list put in the place of another is the one the next call reads."""
+    def one(n):
+        j = {f: torch.zeros(n) for f in ("ao_first", "ao_second", "keep", "mat_Q", "pair_data", "first", "second")}
+        return dict(j, nblk=n, nab=1, count=n)
+    eng.jl = {"ss": one(3), "sp": one(2)}
+    for n in (3, 7):
+        eng.jl["ss"] = one(n)
+        cls, entries, blocks = eng._ket_classes()
+        assert (entries, blocks) == (n + 2, n + 2)
+        assert cls[0].mat_Q == eng.jl["ss"]["mat_Q"].data_ptr() and cls[0].nblk == n
+        assert cls[1].pair_data == eng.jl["sp"]["pair_data"].data_ptr() and cls[1].entry_offset == n

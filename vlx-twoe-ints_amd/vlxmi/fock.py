@@ -8,7 +8,7 @@ factors, K CSR lists, (i,k) lists, Boys tables, assembly indices).  Each
 1. transforms D to the Cartesian AO basis (T^T D T, on the device);
 2. gathers ``mat_D`` for every J pair list, computes the block bounds
    ``beta = max|Q D|`` and orders the ket copy of each list by non-increasing
-   bound (device sort);
+   bound (a rank by counting up to 4096 blocks, a device sort above);
 3. launches the 36 ``computeCoulombFock{AB}{CD}`` and 54
    ``computeExchangeFock{A}{B}{C}{D}`` kernels through the C ABI;
 4. assembles AO J and K from the per-pair outputs and transforms them back
@@ -99,30 +99,30 @@ class FockEngine:
                                I=d.tensor(ik.I.astype(np.uint32)), K=d.tensor(ik.K.astype(np.uint32)),
                                nblk=int(ik.I.size))
         self._build_assembly()
-        self._ket_setup()
-        # AO index sets per angular type (for maxD_bd)
+        # angular type of every Cartesian AO, and AO index sets per type (for maxD_bd)
+        aotype = np.zeros(self.naos, dtype=np.uint8)
+        for p in fl.prims:
+            if p is not None:
+                aotype[p.aoinds.ravel()] = p.l
+        self.ao_type = d.tensor(aotype)
         self.ao_of_type = []
         for p in fl.prims:
             self.ao_of_type.append(d.tensor(np.unique(p.aoinds.ravel()).astype(np.int64)) if p is not None else None)
         self.setup_s = time.time() - t0
 
-    def _ket_setup(self):
-        """The resident Coulomb lists as vlxmi_ket_bounds / vlxmi_ket_order take
-        them, and the angular type of every Cartesian AO."""
+    def _ket_classes(self):
+        """(classes, entries, blocks): the resident Coulomb lists as
+        vlxmi_ket_bounds / vlxmi_ket_order take them, and their total lengths.
+        Made anew for every call, so no address outlives a list in ``jl``."""
         cls = (KetClass * len(self.jl))()
         ent = blk = 0
-        for c, (pc, j) in zip(cls, self.jl.items()):
+        for c, j in zip(cls, self.jl.values()):
             for f in ("ao_first", "ao_second", "keep", "mat_Q", "pair_data", "first", "second"):
                 setattr(c, f, j[f].data_ptr())
             c.nblk, c.entry_offset, c.block_offset, c.nab = j["nblk"], ent, blk, j["nab"]
             ent += j["count"]
             blk += j["nblk"]
-        self._ket_cls, self._ket_entries, self._ket_blocks = cls, ent, blk
-        aotype = np.zeros(self.naos, dtype=np.uint8)
-        for p in self.fl.prims:
-            if p is not None:
-                aotype[p.aoinds.ravel()] = p.l
-        self.ao_type = self.dev.tensor(aotype)
+        return cls, ent, blk
 
     # ------------------------------------------------------------------ assembly
     def _build_assembly(self):
@@ -234,11 +234,11 @@ class FockEngine:
         engine's device whose leading naos x naos part is the Cartesian density."""
         t = self.torch
         Dc = self._kernel_density(Dc)
-        L, st, n = lib(), self.dev.stream_ptr(), self._ket_entries
+        L, st = lib(), self.dev.stream_ptr()
+        cls, n, nblk = self._ket_classes()
         f64 = t.empty((4, n), dtype=t.float64, device=Dc.device)        # mat_D (bra order), then the ket copies
         ints = t.empty((2, n), dtype=t.int32, device=Dc.device)
-        beta = t.empty(self._ket_blocks, dtype=t.float64, device=Dc.device)
-        cls = type(self._ket_cls).from_buffer_copy(self._ket_cls)
+        beta = t.empty(nblk, dtype=t.float64, device=Dc.device)
         if n:
             check(L.vlxmi_ket_bounds(cls, len(cls), Dc.data_ptr(), self.naos, f64[0].data_ptr(), beta.data_ptr(), st), "ket_bounds")
             orders = []
@@ -291,8 +291,8 @@ class FockEngine:
         per ket block (by default the heaviest class's): from 9 on, the chunks
         may be as many times shorter (down to 4 blocks, 2 where even those leave
         SIMDs idle), since a wavefront's time per ket block grows with them and
-        its set-up does not; from 27 on a quarter of the waves is enough.  J of 12 atoms s/p/d 22.8 ms with chunks
-        of 64, 4.2 so; 36 atoms 99.6 and 89.4."""
+        its set-up does not; from 27 on a quarter of the waves is enough.  J of
+        12 atoms s/p/d 22.8 ms with chunks of 64, 4.2 so; 36 atoms 99.6 and 89.4."""
         tiles = max(1, (nbra_blocks + 63) // 64)
         waves = self.target_waves if ncomp < 27 else self.target_waves // 4
         chunk = max(4, min(64, 64 * 9 // ncomp))
