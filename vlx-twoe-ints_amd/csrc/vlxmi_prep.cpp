@@ -88,8 +88,8 @@ ket_bounds_kernel(KetClasses K, const double* __restrict__ D, uint32_t n, double
 // The ket copy of every list: block p of the output is block order[p] of the
 // list, or, without an order (lists of at most VLXMI_KET_RANK_MAX blocks), the
 // block with p others before it by (bound descending, position), which each
-// thread counts for its own block: n^2 / 256 comparisons a wavefront, fewer
-// microseconds than a device sort's launches at this size.
+// thread counts for its own block: n comparisons a thread, fewer microseconds than
+// a device sort's launches at this size.
 __global__ void __launch_bounds__(256)
 ket_order_kernel(KetClasses K, const double* __restrict__ beta, const double* __restrict__ mat_D,
                  uint32_t* __restrict__ first, uint32_t* __restrict__ second, double* __restrict__ pair_data,

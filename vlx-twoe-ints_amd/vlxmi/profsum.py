@@ -117,7 +117,7 @@ def counters_markdown(pmc_dir, per_class_path, top=25, copy_bytes=512 << 20):
     def by_name(d):
         out = {}
         for (_, name), v in d.items():
-            out.setdefault(name, v)
+            out.setdefault(name[:-3] if name.endswith("_ks") else name, v)      # ket-split launches
         return out
 
     mem, fe, wr = by_name(mem), by_name(fe), by_name(wr)
@@ -190,6 +190,9 @@ def busy_markdown(path, top=30):
 
     * VALU busy: SQ_ACTIVE_INST_VALU / SQ_WAVE_CYCLES, the share of a wave's
       life spent issuing vector ALU instructions;
+    * VALU / clk / CU: SQ_INSTS_VALU over the clocks of all CUs,
+      (GRBM_GUI_ACTIVE / 8 XCDs) x 256; a CU issues at most one 64-lane FP64
+      instruction a clock;
     * waiting: SQ_WAIT_INST_ANY / SQ_WAVE_CYCLES, the share spent waiting for
       any instruction's inputs (memory, mostly);
     * TA / TD busy: summed over the per-CU units, divided by
@@ -203,17 +206,18 @@ def busy_markdown(path, top=30):
             a[k] = a.get(k, 0.0) + x
     rows = sorted(agg.items(), key=lambda kv: -kv[1].get("_t", 0.0))[:top]
     o = ["| kernel | dispatches | ms / dispatch | waves | VALU instr / wave | VMEM rd / wave | LDS instr / wave "
-         "| VALU busy | waiting | TA busy | TD busy |",
-         "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
+         "| VALU busy | VALU / clk / CU | waiting | TA busy | TD busy |",
+         "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
     for name, a in rows:
         n = a["_n"]
         w = a.get("SQ_WAVES", 0.0) or 1.0
         cyc = a.get("SQ_WAVE_CYCLES", 0.0) or 1.0
         g = a.get("GRBM_GUI_ACTIVE", 0.0) / 8.0 * 256.0
-        o.append("| %s | %d | %.3f | %.0f | %.1f | %.2f | %.2f | %.2f | %.2f | %.2f | %.2f |" % (
+        o.append("| %s | %d | %.3f | %.0f | %.1f | %.2f | %.2f | %.2f | %.2f | %.2f | %.2f | %.2f |" % (
             name, n, 1e3 * a.get("_t", 0.0) / n, w / n, a.get("SQ_INSTS_VALU", 0.0) / w,
             a.get("SQ_INSTS_VMEM_RD", 0.0) / w, a.get("SQ_INSTS_LDS", 0.0) / w,
-            a.get("SQ_ACTIVE_INST_VALU", 0.0) / cyc, a.get("SQ_WAIT_INST_ANY", 0.0) / cyc,
+            a.get("SQ_ACTIVE_INST_VALU", 0.0) / cyc, a.get("SQ_INSTS_VALU", 0.0) / g if g else 0.0,
+            a.get("SQ_WAIT_INST_ANY", 0.0) / cyc,
             a.get("TA_TA_BUSY", 0.0) / g if g else 0.0, a.get("TD_TD_BUSY", 0.0) / g if g else 0.0))
     return "\n".join(o) + "\n"
 
